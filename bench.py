@@ -36,11 +36,18 @@ HBM_PEAK_GBS = 8000.0
 #             (4 bytes) + 3 faces (8 bytes), write 9 prim + 3 faces (4 bytes);
 #             FP32C corrector: read 6 hi + 6 lo + 18 fluxes + 3 EMFs (4 bytes)
 #             + 3 faces (8 bytes), write 6 hi + 6 lo + 9 prim (4) + 3 faces (8)
+#   stage_*:  per cell, a fused stage.  Predictor: read 9 prim + 3 faces
+#             (FP32C also 6 hi words), write the same; corrector: read the
+#             predictor's and the step's, write 9 prim + 3 faces (FP32C:
+#             9 prim, 6 hi, 6 lo words and 3 faces)
 KERNEL_BYTES = {
-    "fp64": {"flux": 18 * 8, "emf": 15 * 8, "update_pred": 45 * 8, "update_corr": 45 * 8},
-    "fp64fma": {"flux": 18 * 8, "emf": 15 * 8, "update_pred": 45 * 8, "update_corr": 45 * 8},
+    "fp64": {"flux": 18 * 8, "emf": 15 * 8, "update_pred": 45 * 8, "update_corr": 45 * 8,
+             "stage_pred": 24 * 8, "stage_corr": 36 * 8},
+    "fp64fma": {"flux": 18 * 8, "emf": 15 * 8, "update_pred": 45 * 8, "update_corr": 45 * 8,
+                "stage_pred": 24 * 8, "stage_corr": 36 * 8},
     "fp32c": {"flux": 18 * 4, "emf": 15 * 4, "update_pred": 48 * 4 + 3 * 8,
-              "update_corr": 54 * 4 + 6 * 8},
+              "update_corr": 54 * 4 + 6 * 8, "stage_pred": 27 * 4 + 3 * 8,
+              "stage_corr": 45 * 4 + 6 * 8},
 }
 # HBM bytes per launch of the dominant kernels at 256^3 (FETCH_SIZE x 2.0 +
 # WRITE_SIZE x 1.0, scaled by a plain device copy) and the fraction of the

@@ -10,6 +10,9 @@ keeps the candidate with the smallest summed time:
   flux   -- Godunov fluxes of both stages (all directions in one launch)
   emf    -- edge EMF kernels
   update -- stage updates (the corrector carries the fused CFL reduction)
+Shape 0 in all three classes runs large grids' stages as fused passes
+("stage"), which replace all three; they are kept where they take less time
+than the best separate kernels together.
 The runs advance the context's state: callers tune first and then upload
 their initial state again, or tune a scratch context of the same shape.
 """
@@ -20,8 +23,10 @@ BATCH_CANDIDATES = (2048, 4096, 8192, 16384, 65536)
 
 
 def _class_times(kt):
-    out = {"flux": 0.0, "emf": 0.0, "update": 0.0}
+    out = {"flux": 0.0, "emf": 0.0, "update": 0.0, "stage": 0.0}
     for name, (tot, n) in kt.items():
+        if name.startswith("stage"):
+            out["stage"] += tot
         if name.startswith("flux"):
             out["flux"] += tot
         elif name.startswith("emf"):
@@ -58,7 +63,14 @@ def autotune(ctx, steps=2, candidates=CANDIDATES, passes=2):
             ctx.set_kernel_timing(False)
             t = _class_times(ctx.kernel_timing())
             table[c] = t if c not in table else {k: min(v, table[c][k]) for k, v in t.items()}
-    best = tuple(min(candidates, key=lambda c: table[c][k]) for k in ("flux", "emf", "update"))
+    kinds = ("flux", "emf", "update")
+    fused = [c for c in candidates if table[c]["stage"] > 0.0]
+    separate = [c for c in candidates if c not in fused]
+    best = (0, 0, 0)
+    if separate:
+        best = tuple(min(separate, key=lambda c: table[c][k]) for k in kinds)
+        if fused and table[fused[0]]["stage"] <= sum(table[c][k] for c, k in zip(best, kinds)):
+            best = (fused[0],) * 3
     ctx.set_tuning(*best)
     return best, table
 

@@ -294,20 +294,30 @@ __device__ __forceinline__ double cds_cell_g(const GM &gm, const Geo &g, const d
     double cds = fmax(fmax(cx / gm.dlf(0, i), cy / gm.dlf(1, j)), cz / gm.dlf(2, k));
     return (cds > 0.) ? cds : 0.;
   }
+  if (fms_ref) {  // one fast speed for every axis
+    const double a = fms(wv, g.gam);
+    const double cx = fabs(wv[VX]) + a;
+    const double cy = g.dims >= 2 ? fabs(wv[VY]) + a : 0.;
+    const double cz = g.dims >= 3 ? fabs(wv[VZ]) + a : 0.;
+    const double cds = fmax(fmax(cx / gm.dlf(0, i), cy / gm.dlf(1, j)), cz / gm.dlf(2, k));
+    return (cds > 0.) ? cds : 0.;
+  }
   const double cx = fabs(wv[VX]) + fms(wv, g.gam);
   double cy = 0., cz = 0.;
   if (g.dims >= 2) {
     double wy[NMODE];
 #pragma unroll
     for (int n = 0; n < NMODE; ++n) wy[n] = wv[n];
-    if (!fms_ref) { wy[BX] = wv[BY]; wy[BY] = wv[BX]; }
+    wy[BX] = wv[BY];
+    wy[BY] = wv[BX];
     cy = fabs(wv[VY]) + fms(wy, g.gam);
   }
   if (g.dims >= 3) {
     double wz[NMODE];
 #pragma unroll
     for (int n = 0; n < NMODE; ++n) wz[n] = wv[n];
-    if (!fms_ref) { wz[BX] = wv[BZ]; wz[BZ] = wv[BX]; }
+    wz[BX] = wv[BZ];
+    wz[BZ] = wv[BX];
     cz = fabs(wv[VZ]) + fms(wz, g.gam);
   }
   double cds = fmax(fmax(cx / gm.dlf(0, i), cy / gm.dlf(1, j)), cz / gm.dlf(2, k));
@@ -337,6 +347,7 @@ struct bnz_ctx {
   int nt[3] = {1, 1, 1};
   int i1, i2, j1, j2, k1, k2;
   long ncell = 0;
+  int ncu = 256;  // compute units of the device
   hipStream_t stream = nullptr;
   double *w = nullptr, *ws = nullptr, *b = nullptr, *bs = nullptr;
   double *fx = nullptr, *fy = nullptr, *fz = nullptr, *ee = nullptr;
@@ -346,10 +357,11 @@ struct bnz_ctx {
   // bnz_advance: a captured chunk of steps, replayed while the buffers,
   // CFL partial count and work shapes it was captured with are current
   struct ChunkKey {
-    const void *w, *ws, *b, *bs, *part;
+    const void *w, *ws, *b, *bs, *ee, *part;
     int dt_parts, flux_chunk, emf_chunk, update_chunk;
     bool operator==(const ChunkKey &o) const {
-      return w == o.w && ws == o.ws && b == o.b && bs == o.bs && part == o.part &&
+      return w == o.w && ws == o.ws && b == o.b && bs == o.bs && ee == o.ee &&
+             part == o.part &&
              dt_parts == o.dt_parts && flux_chunk == o.flux_chunk &&
              emf_chunk == o.emf_chunk && update_chunk == o.update_chunk;
     }

@@ -610,7 +610,7 @@ struct StatePart {
 // bnz_advance's captured chunk: its key and its release
 bnz_ctx::ChunkKey chunk_key(const bnz_ctx *c) {
   return bnz_ctx::ChunkKey{c->w,          c->ws,         c->b,
-                           c->bs,         c->part,       c->dt_parts,
+                           c->bs,         c->ee,         c->part,       c->dt_parts,
                            c->flux_chunk, c->emf_chunk,  c->update_chunk};
 }
 void drop_chunk_graph(bnz_ctx *c) {
@@ -812,6 +812,7 @@ int bnz_create(const bnz_params *p, bnz_ctx **out) {
     if (rc) return rc;
   }
   if (hipSetDevice(p->device) != hipSuccess) return fail(c, BNZ_EHIP, "hipSetDevice failed");
+  HIPCHK(c, hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, p->device));
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   HIPCHK(c, hipHostMalloc(&c->hbuf, 8 * sizeof(double), hipHostMallocDefault));
   for (int q = 0; q < 2; ++q) HIPCHK(c, hipEventCreateWithFlags(&c->hev[q], hipEventDisableTiming));
@@ -878,6 +879,7 @@ int bnz_create(const bnz_params *p, bnz_ctx **out) {
     }
     c->npart_cap = std::max({(long)blocks_for(a.total()) * std::max(NDIAG, NHIST) + 64,
                              (long)blocks_for(c->ncell), (long)tiled_blocks(grid, 1, 2),
+                             c->dims >= 2 ? tile_parts(c) : 0L,
                              (long)(c->nt[0] + STEP1_CELLS - 1) / STEP1_CELLS});
   }
   HIPCHK(c, hipMalloc(&c->part, c->npart_cap * sizeof(double)));

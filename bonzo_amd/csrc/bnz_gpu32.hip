@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "bnz_kern32.hpp"
+#include "bnz_tile32.hpp"
 
 using namespace bnz;
 
@@ -109,6 +110,72 @@ __global__ __launch_bounds__(BLK) void k32_update_corr(Geo g, Corr32 a, Lims L,
     cdsmax = update32_corr<DIMS, typename std::conditional<UG, GeoUni, GeoArr>::type, FLY>(
         g, a, L, dts, act, fms_ref, i, j, k, we, wl);
   block_max_to(cdsmax, part);
+}
+
+// One FP32C stage of a 2D grid, a tile per workgroup (as the FP64 k_stage2).
+template <bool PRED, int ORDER, int RS, int TX, int TY, typename BF>
+__global__ __launch_bounds__(TX *TY, TX *TY >= 512 ? 4 : 2) void k32_stage2(Geo g, const float *__restrict__ wf,
+                                                     const BF *__restrict__ bf, Pred32 ap,
+                                                     Corr32 ac, Lims L, Tiling tl, Box act,
+                                                     Bnd bnd, Walls wl, int fms_ref, double *dev,
+                                                     DtFold dtf, double *__restrict__ part,
+                                                     int *nguard) {
+  constexpr int NT = TX * TY;
+  __shared__ float lds[tile2_lds32<NT>()];
+  const StepDt<NT> sd(dtf, dev);  // (the corrector has no fold: dev[0])
+  if (sd.past(dtf)) {  // a step past t_max: state unchanged, faces carried over
+    if (PRED && blockIdx.x == 0 && threadIdx.x == 0) dev[0] = 0.;
+    if (!PRED)
+      for (long c = (long)blockIdx.x * NT + threadIdx.x; c < g.sv; c += (long)gridDim.x * NT)
+        for (int a = 0; a < 3; ++a) ac.b1[a * g.sv + c] = ac.b[a * g.sv + c];
+    return;
+  }
+  if (!PRED) time_advance_once(dev);
+  int ng = 0;
+  const int b = (int)xcd_block();
+  const double cds = stage2_tile32<PRED, ORDER, RS, TX, TY>(
+      g, wf, bf, ap, ac, L, [&] { return sd.value(dtf, dev); }, act, bnd, wl, fms_ref,
+      tl.o[0] + (b % tl.n[0]) * (TX - 2), tl.o[1] + (b / tl.n[0]) * (TY - 2), lds, ng);
+  if (!PRED) {
+    const double m = block_max_nt<NT>(cds);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+  }
+  if (ng) atomicAdd(nguard, ng);
+}
+
+// One FP32C stage of a 3D grid (as the FP64 k_stage3).
+template <bool PRED, int ORDER, int RS, bool UG, int TX, int TY, typename BF>
+__global__ __launch_bounds__(TX *TY, STAGE3_PER_CU) void k32_stage3(
+    Geo g, const float *__restrict__ wf, const BF *__restrict__ bf, Pred32 ap, Corr32 ac, Lims L,
+    Tiling3 tl, Box act, Walls wl, int fms_ref, double *dev, DtFold dtf, double *__restrict__ part,
+    int *nguard) {
+  constexpr int NT = TX * TY;
+  using R = typename std::conditional<PRED, float, double>::type;
+  __shared__ float lds[NSLOT3_32 * NT];
+  __shared__ R ldu[NSLOT3_U * NT];
+  const StepDt<NT> sd(dtf, dev);
+  if (sd.past(dtf)) {  // a step past t_max: state unchanged, faces carried over
+    if (PRED && blockIdx.x == 0 && threadIdx.x == 0) dev[0] = 0.;
+    if (!PRED)
+      for (long c = (long)blockIdx.x * NT + threadIdx.x; c < g.sv; c += (long)gridDim.x * NT)
+        for (int a = 0; a < 3; ++a) ac.b1[a * g.sv + c] = ac.b[a * g.sv + c];
+    return;
+  }
+  const double dt = sd.value(dtf, dev);
+  int b = (int)(tl.runs ? run_block() : xcd_block());
+  const int bx = b % tl.n[0];
+  b /= tl.n[0];
+  const int by = b % tl.n[1], kb = tl.o[2] + b / tl.n[1] * tl.nz;
+  int ng = 0;
+  using GM = typename std::conditional<UG, GeoUni, GeoArr>::type;
+  const double cds = stage3_column32<PRED, ORDER, RS, GM, TX, TY>(
+      g, wf, bf, ap, ac, L, dt, act, wl, fms_ref, tl.o[0] + bx * (TX - 2),
+      tl.o[1] + by * (TY - 2), kb, min(kb + tl.nz - 1, tl.top), lds, ldu, ng);
+  if (!PRED) {
+    const double m = block_max_nt<NT>(cds);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+  }
+  if (ng) atomicAdd(nguard, ng);
 }
 
 // One FP32C stage of a 1D grid in one pass (stage32_cell): workgroup b owns
@@ -381,7 +448,77 @@ void stage32(bnz_ctx *c, int order, const Lims &L) {
   }
 }
 
+// A 2D FP32C step as two launches (as the FP64 stage2_launch): w32, b -> ws32,
+// bs32 -> uh, ul, w32 in place and the faces to bs.
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+void stage2_launch32(bnz_ctx *c, const Lims &L) {
+  const Tiling tl = tiling2(c, L, PRED, TX - 2, TY - 2);
+  const DtFold dtf = PRED ? take_dt(c) : DtFold{};
+  const Pred32 ap{c->w32, c->uh, c->b, c->fx32, c->fy32, c->fz32, c->ee32, c->bs32, c->ws32};
+  const Corr32 ac{c->uh, c->ul, c->b, c->fx32, c->fy32, c->fz32, c->ee32, c->bs, c->w32};
+  Launch t(c, PRED ? "stage_pred" : "stage_corr");
+  using BF = typename std::conditional<PRED, double, float>::type;
+  const BF *bf;
+  if constexpr (PRED) bf = c->b;
+  else bf = c->bs32;
+  hipLaunchKernelGGL((k32_stage2<PRED, ORDER, RS, TX, TY, BF>), dim3(tl.blocks()), dim3(TX * TY),
+                     0, c->stream, c->g, PRED ? c->w32 : c->ws32, bf, ap, ac, L, tl,
+                     active_box(c), bnd_of(c), walls32(c), c->p.dt_fms_ref, c->dev, dtf, c->part,
+                     (int *)(c->dev + 4));
+  c->dt_parts = PRED ? 0 : tl.blocks();
+}
+
+// A 3D FP32C step as two launches and the ghost fill.
+template <bool PRED, int ORDER, int RS>
+void stage3_launch32(bnz_ctx *c, const Lims &L) {
+  constexpr int TX = TILE3[0], TY = TILE3[1];
+  // the corrector walks every cell whose faces the stage solves, so that each
+  // guarded face is counted
+  const Tiling3 tl = tiling3(c, L, PRED, false, TX - 2, TY - 2);
+  const DtFold dtf = PRED ? take_dt(c) : DtFold{};
+  const Pred32 ap{c->w32, c->uh, c->b, c->fx32, c->fy32, c->fz32, c->ee32, c->bs32, c->ws32};
+  const Corr32 ac{c->uh, c->ul, c->b, c->fx32, c->fy32, c->fz32, c->ee32, c->bs, c->w32};
+  Launch t(c, PRED ? "stage_pred" : "stage_corr");
+  using BF = typename std::conditional<PRED, double, float>::type;
+  const BF *bf;
+  if constexpr (PRED) bf = c->b;
+  else bf = c->bs32;
+#define STAGE3_ARGS32                                                                          \
+  dim3(tl.blocks()), dim3(TX *TY), 0, c->stream, c->g, PRED ? c->w32 : c->ws32, bf, ap, ac, L,  \
+      tl, active_box(c), walls32(c), c->p.dt_fms_ref, c->dev, dtf, c->part, (int *)(c->dev + 4)
+  if (c->g.unif)
+    hipLaunchKernelGGL((k32_stage3<PRED, ORDER, RS, true, TX, TY, BF>), STAGE3_ARGS32);
+  else
+    hipLaunchKernelGGL((k32_stage3<PRED, ORDER, RS, false, TX, TY, BF>), STAGE3_ARGS32);
+#undef STAGE3_ARGS32
+  c->dt_parts = PRED ? 0 : tl.blocks();
+}
+
+template <bool PRED, int ORDER>
+void stage_fused32(bnz_ctx *c, const Lims &L) {
+  const bool small = c->ncell <= TILE2_SMALL_CELLS, hlld = c->p.rsolver == BNZ_RS_HLLD;
+  if (c->dims == 3) {
+    if (hlld) stage3_launch32<PRED, ORDER, BNZ_RS_HLLD>(c, L);
+    else stage3_launch32<PRED, ORDER, BNZ_RS_HLL>(c, L);
+  } else if (hlld) {
+    if (small) stage2_launch32<PRED, ORDER, BNZ_RS_HLLD, TILE2_SMALL[0], TILE2_SMALL[1]>(c, L);
+    else stage2_launch32<PRED, ORDER, BNZ_RS_HLLD, TILE2_BIG[0], TILE2_BIG[1]>(c, L);
+  } else {
+    if (small) stage2_launch32<PRED, ORDER, BNZ_RS_HLL, TILE2_SMALL[0], TILE2_SMALL[1]>(c, L);
+    else stage2_launch32<PRED, ORDER, BNZ_RS_HLL, TILE2_BIG[0], TILE2_BIG[1]>(c, L);
+  }
+}
+
 void f32_step_body(bnz_ctx *c) {
+  if (fused_stages(c)) {  // 2D: ghosts and time included
+    if (c->pdt_pending && c->pdt.npart > DT_PARTS_IN_STAGE) flush_dt(c);
+    stage_fused32<true, 0>(c, integr_lims(c, 0));
+    if (c->order) stage_fused32<false, 1>(c, integr_lims(c, 1));
+    else stage_fused32<false, 0>(c, integr_lims(c, 0));
+    std::swap(c->b, c->bs);
+    if (c->dims == 3) ghost32(c, true);  // and the time advance
+    return;
+  }
   if (c->dims == 1) {  // fluxes through LDS
     stage32<true>(c, 0, integr_lims(c, 0));
     stage32<false>(c, c->order, integr_lims(c, c->order));

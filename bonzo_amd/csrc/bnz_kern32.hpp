@@ -396,13 +396,20 @@ struct Corr32 {
 // returns the CFL speed of the new state (0 outside the active cells).  Operands loaded up front as in the
 // predictor.
 // SPLIT (the corrector of a fused 1D step): the new hi and lo words go to
-// uh1 and ul1 instead of back to a.uh and a.ul.
-template <int DIMS, class GM, class FL, class EM, bool SPLIT = false>
+// uh1 and ul1 instead of back to a.uh and a.ul.  copy gets the new hi words,
+// prim and lower faces of an updated cell (the ghost images).  lo_only: a
+// ghost cell whose other words come from the fill in the same launch.
+struct NoCopy32 {
+  __device__ __forceinline__ void operator()(const float *, const double *, const double *) const {}
+};
+template <int DIMS, class GM, class FL, class EM, bool SPLIT = false, class COPY = NoCopy32>
 __device__ __forceinline__ double update32_corr_e(const Geo &g, const Corr32 &a, const Lims &L,
                                                   const double *__restrict__ dts, const Box &act,
                                                   int fms_ref, const FL &fl, const EM &em, int i,
                                                   int j, int k, float *uh1 = nullptr,
-                                                  float *ul1 = nullptr) {
+                                                  float *ul1 = nullptr,
+                                                  const COPY &copy = COPY{},
+                                                  bool lo_only = false) {
   const long c = ((long)k * g.nt[1] + j) * g.nt[0] + i, sv = g.sv;
   double cdsmax = 0.;
   const double dt = dts[0];
@@ -450,6 +457,13 @@ __device__ __forceinline__ double update32_corr_e(const Geo &g, const Corr32 &a,
   else
     u[BZ] = lo[2];
   cons2prim(wv, u, g.gam);
+  if (lo_only) {
+    if (ro.cell) {
+#pragma unroll
+      for (int n = 0; n < NMODE - 3; ++n) a.ul[n * sv + c] = nl[n];
+    }
+    return 0.;
+  }
   if (ro.fX) a.b1[c] = lo[0];
   if (ro.fY) a.b1[sv + c] = lo[1];
   if (ro.fZ) a.b1[2 * sv + c] = lo[2];
@@ -461,6 +475,7 @@ __device__ __forceinline__ double update32_corr_e(const Geo &g, const Corr32 &a,
     }
 #pragma unroll
     for (int n = 0; n < NMODE; ++n) a.w32[n * sv + c] = (float)wv[n];
+    copy(nh, wv, lo);
     if (i >= act.lo[0] && i < act.lo[0] + act.n[0] && j >= act.lo[1] &&
         j < act.lo[1] + act.n[1] && k >= act.lo[2] && k < act.lo[2] + act.n[2])
       cdsmax = cds_cell_g(gm, g, wv, fms_ref, i, j, k);

@@ -9,6 +9,17 @@
 
 namespace bnz {
 
+// The Riemann solver RS on one face; 0 if no region matched.
+template <int RS>
+__device__ __forceinline__ int solve_face(double *f, const double *wl, const double *wr, double gam,
+                                          double gamm1i) {
+  if (RS == BNZ_RS_HLLD) return flux_hlld(f, wl, wr, gam, gamm1i);
+  if (RS == BNZ_RS_HLLT) return flux_hllt(f, wl, wr, gam, gamm1i);
+  if (RS == BNZ_RS_HLLC) return flux_hllc(f, wl, wr, gam, gamm1i);
+  if (RS == RS_HLL_HYDRO) return flux_hll<double, true>(f, wl, wr, gam, gamm1i);
+  return flux_hll(f, wl, wr, gam, gamm1i);
+}
+
 // Godunov fluxes of one direction (godunov.pyx:20-210 with the double-buffered
 // left state of D1).  Face index c is the lower face of cell c, between cells
 // c-1 and c.  The flux is stored in global variable order, flux[n][c], except
@@ -66,17 +77,7 @@ __device__ __forceinline__ void flux_face_to(const Geo &g, const double *__restr
   wr[BX] = bn;
 
   double f[NMODE];
-  int reg;
-  if (RS == BNZ_RS_HLLD)
-    reg = flux_hlld(f, wl, wr, g.gam, g.gamm1i);
-  else if (RS == BNZ_RS_HLLT)
-    reg = flux_hllt(f, wl, wr, g.gam, g.gamm1i);
-  else if (RS == BNZ_RS_HLLC)
-    reg = flux_hllc(f, wl, wr, g.gam, g.gamm1i);
-  else if (RS == RS_HLL_HYDRO)
-    reg = flux_hll<double, true>(f, wl, wr, g.gam, g.gamm1i);
-  else
-    reg = flux_hll(f, wl, wr, g.gam, g.gamm1i);
+  const int reg = solve_face<RS>(f, wl, wr, g.gam, g.gamm1i);
   if (reg == 0) return;  // reference leaves the flux row untouched
   sink(f, c);
 }
@@ -325,16 +326,24 @@ struct EmfLds1D {  // the 1D EMFs from the LDS fluxes
   }
 };
 
+// What the update does with a cell's new prim and lower faces besides
+// storing them: nothing.
+struct NoCopy {
+  __device__ __forceinline__ void operator()(const double *, double, double, double) const {}
+};
+
 // LDS_OUT (predictor of a fused 1D step): the new prim goes to the LDS
-// array w1 as w1[n * BLK + lslot] and no face is stored (b1 unused).
-template <int DIMS, bool PRED, bool DTRED, class EMF, class GM, class FL, bool LDS_OUT = false>
+// array w1 as w1[n * BLK + lslot] and no face is stored (b1 unused).  copy
+// gets the new prim and lower faces of an updated cell (the ghost images).
+template <int DIMS, bool PRED, bool DTRED, class EMF, class GM, class FL, bool LDS_OUT = false,
+          class COPY = NoCopy>
 __device__ __forceinline__ double update_cell_e(const Geo &g, const GM &gm, const double *w0,
                                                 const FL &fl, const EMF &em,
                                                 const double *__restrict__ b0,
                                                 double *__restrict__ b1, double *w1,
                                                 const Lims &L, const double *__restrict__ dts,
                                                 const Box &act, int fms_ref, int i, int j, int k,
-                                                int lslot = 0) {
+                                                int lslot = 0, const COPY &copy = COPY{}) {
   const long c = ((long)k * g.nt[1] + j) * g.nt[0] + i;
   const long sv = g.sv;
   const double dt = PRED ? 0.5 * dts[0] : dts[0];
@@ -465,6 +474,7 @@ __device__ __forceinline__ double update_cell_e(const Geo &g, const GM &gm, cons
   if (cell) {
 #pragma unroll
     for (int n = 0; n < NMODE; ++n) w1[n * sv + c] = wn[n];
+    copy(wn, bxl, byl, bzl);
   } else if (PRED) {
 #pragma unroll
     for (int n = 0; n < NMODE; ++n) w1[n * sv + c] = wv[n];

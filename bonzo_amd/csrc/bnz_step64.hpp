@@ -17,6 +17,7 @@
 
 #include "bnz_kern64.hpp"
 #include "bnz_rk3.hpp"
+#include "bnz_tile64.hpp"
 
 namespace {
 
@@ -182,9 +183,128 @@ __global__ __launch_bounds__(BLK) void k_update(Geo g, const double *w0, const d
   if (DTRED) block_max_to(cdsmax, part);
 }
 
+// One stage of a 2D grid, a tile per workgroup (stage2_tile).  The predictor
+// finds the step's dt (step_dt); the corrector leaves the CFL partial of its
+// tile, writes the ghosts and advances the time, so that a step is two
+// launches.
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+__global__ __launch_bounds__(TX *TY, TX *TY >= 512 ? 4 : 2) void k_stage2(Geo g, const double *__restrict__ wf,
+                                                   const double *__restrict__ bf,
+                                                   const double *w0, const double *b0, double *w1,
+                                                   double *b1, Lims L, Tiling tl, Box act,
+                                                   Bnd bnd, int fms_ref, double *dev, DtFold dtf,
+                                                   double *__restrict__ part) {
+  constexpr int NT = TX * TY;
+  __shared__ double lds[tile2_lds<NT>()];
+  const StepDt<NT> sd(dtf, dev);  // (the corrector has no fold: dev[0])
+  if (sd.past(dtf)) {  // a step past t_max: state unchanged, faces carried over
+    if (PRED && blockIdx.x == 0 && threadIdx.x == 0) dev[0] = 0.;
+    if (!PRED)
+      for (long c = (long)blockIdx.x * NT + threadIdx.x; c < g.sv; c += (long)gridDim.x * NT)
+        for (int a = 0; a < 3; ++a) b1[a * g.sv + c] = b0[a * g.sv + c];
+    return;
+  }
+  if (!PRED) time_advance_once(dev);  // nothing else in this launch reads t
+  const int b = (int)xcd_block();
+  const double cds = stage2_tile<PRED, ORDER, RS, TX, TY>(
+      g, wf, bf, w0, b0, w1, b1, L, [&] { return sd.value(dtf, dev); }, act, bnd, fms_ref,
+      tl.o[0] + (b % tl.n[0]) * (TX - 2), tl.o[1] + (b / tl.n[0]) * (TY - 2), lds);
+  if (!PRED) {
+    const double m = block_max_nt<NT>(cds);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+  }
+}
+
+// One stage of a 3D grid, a run of planes of a column of tiles per workgroup
+// (stage3_column); otherwise as k_stage2, but the ghosts are filled by a
+// launch of their own.
+template <bool PRED, int ORDER, int RS, bool UG, int TX, int TY>
+__global__ __launch_bounds__(TX *TY, STAGE3_PER_CU) void k_stage3(Geo g, const double *__restrict__ wf,
+                                                       const double *__restrict__ bf,
+                                                       const double *w0,
+                                                       const double *__restrict__ b0, double *w1,
+                                                       double *b1, Lims L, Tiling3 tl, Box act,
+                                                       int fms_ref, double *dev, DtFold dtf,
+                                                       double *__restrict__ part) {
+  constexpr int NT = TX * TY;
+  __shared__ double lds[NSLOT3 * NT];
+  const StepDt<NT> sd(dtf, dev);
+  if (sd.past(dtf)) {  // a step past t_max: state unchanged, faces carried over
+    if (PRED && blockIdx.x == 0 && threadIdx.x == 0) dev[0] = 0.;
+    if (!PRED)
+      for (long c = (long)blockIdx.x * NT + threadIdx.x; c < g.sv; c += (long)gridDim.x * NT)
+        for (int a = 0; a < 3; ++a) b1[a * g.sv + c] = b0[a * g.sv + c];
+    return;
+  }
+  const double dt = sd.value(dtf, dev);
+  int b = (int)(tl.runs ? run_block() : xcd_block());
+  const int bx = b % tl.n[0];
+  b /= tl.n[0];
+  const int by = b % tl.n[1], kb = tl.o[2] + b / tl.n[1] * tl.nz;
+  using GM = typename std::conditional<UG, GeoUni, GeoArr>::type;
+  const double cds = stage3_column<PRED, ORDER, RS, GM, TX, TY>(
+      g, wf, bf, w0, b0, w1, b1, L, dt, act, fms_ref, tl.o[0] + bx * (TX - 2), tl.o[1] + by * (TY - 2),
+      kb, min(kb + tl.nz - 1, tl.top), lds);
+  if (!PRED) {
+    const double m = block_max_nt<NT>(cds);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+  }
+}
+
 // ==========================================================================
 // Launches
 // ==========================================================================
+
+// A 2D step as two launches: w, b -> ws, bs -> w, ee (the face buffer the
+// caller swaps with b; no EMF array is needed here).
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+void stage2_launch(bnz_ctx *c, const Lims &L) {
+  const Tiling tl = tiling2(c, L, PRED, TX - 2, TY - 2);
+  const DtFold dtf = PRED ? take_dt(c) : DtFold{};
+  Launch t(c, PRED ? "stage_pred" : "stage_corr");
+  hipLaunchKernelGGL((k_stage2<PRED, ORDER, RS, TX, TY>), dim3(tl.blocks()), dim3(TX * TY), 0,
+                     c->stream, c->g, PRED ? c->w : c->ws, PRED ? c->b : c->bs, c->w, c->b,
+                     PRED ? c->ws : c->w, PRED ? c->bs : c->ee, L, tl, active_box(c), bnd_of(c),
+                     cfl_mode(c), c->dev, dtf, c->part);
+  c->dt_parts = PRED ? 0 : tl.blocks();
+}
+
+// A 3D step as two launches, buffers as stage2_launch
+template <bool PRED, int ORDER, int RS>
+void stage3_launch(bnz_ctx *c, const Lims &L) {
+  constexpr int TX = TILE3[0], TY = TILE3[1];
+  const Tiling3 tl = tiling3(c, L, PRED, true, TX - 2, TY - 2);
+  const DtFold dtf = PRED ? take_dt(c) : DtFold{};
+  Launch t(c, PRED ? "stage_pred" : "stage_corr");
+#define STAGE3_ARGS                                                                             \
+  dim3(tl.blocks()), dim3(TX *TY), 0, c->stream, c->g, PRED ? c->w : c->ws,                    \
+      PRED ? c->b : c->bs, c->w, c->b, PRED ? c->ws : c->w, PRED ? c->bs : c->ee, L, tl,        \
+      active_box(c), cfl_mode(c), c->dev, dtf, c->part
+  if (c->g.unif)
+    hipLaunchKernelGGL((k_stage3<PRED, ORDER, RS, true, TX, TY>), STAGE3_ARGS);
+  else
+    hipLaunchKernelGGL((k_stage3<PRED, ORDER, RS, false, TX, TY>), STAGE3_ARGS);
+#undef STAGE3_ARGS
+  c->dt_parts = PRED ? 0 : tl.blocks();
+}
+
+template <bool PRED, int ORDER>
+void stage_fused(bnz_ctx *c, const Lims &L) {
+  const bool small = c->ncell <= TILE2_SMALL_CELLS;
+  const int rs = rs_kern(c);
+#define FUSED(RS)                                              \
+  do {                                                          \
+    if (c->dims == 3) stage3_launch<PRED, ORDER, RS>(c, L);     \
+    else if (small) stage2_launch<PRED, ORDER, RS, TILE2_SMALL[0], TILE2_SMALL[1]>(c, L);     \
+    else stage2_launch<PRED, ORDER, RS, TILE2_BIG[0], TILE2_BIG[1]>(c, L);          \
+  } while (0)
+  if (rs == BNZ_RS_HLLD) FUSED(BNZ_RS_HLLD);
+  else if (rs == BNZ_RS_HLLT) FUSED(BNZ_RS_HLLT);
+  else if (rs == BNZ_RS_HLLC) FUSED(BNZ_RS_HLLC);
+  else if (rs == RS_HLL_HYDRO) FUSED(RS_HLL_HYDRO);
+  else FUSED(BNZ_RS_HLL);
+#undef FUSED
+}
 
 template <int ORDER, int RS, bool CP>
 void launch_fluxes_cp(bnz_ctx *c, const double *w, const double *bf, const Lims &L) {
@@ -390,6 +510,15 @@ void launch_step_body(bnz_ctx *c) {
   }
   Lims L0 = integr_lims(c, 0);
   Lims L1 = integr_lims(c, c->order);
+  if (fused_stages(c)) {  // 2D: ghosts and time included
+    if (c->pdt_pending && c->pdt.npart > DT_PARTS_IN_STAGE) flush_dt(c);
+    stage_fused<true, 0>(c, L0);
+    if (c->order) stage_fused<false, 1>(c, L1);
+    else stage_fused<false, 0>(c, L1);
+    std::swap(c->b, c->ee);
+    if (c->dims == 3) launch_ghost_step64(c);  // and the time advance
+    return;
+  }
   if (c->dims == 1) {  // the whole step through LDS
     launch_step1(c, L0, L1);
   } else {

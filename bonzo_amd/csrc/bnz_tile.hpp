@@ -1,0 +1,394 @@
+// bnz_tile.hpp -- pieces shared by the fused stage kernels (bnz_tile64.hpp,
+// bnz_tile32.hpp), which form a stage's fluxes, EMFs and update in one pass
+// over a tile: the dt of the step, the CFL maximum of a workgroup, and the
+// ghost images of an active cell.
+#pragma once
+#include "bnz_common.hpp"
+
+namespace bnz {
+
+// The dt of a step, by every workgroup of its first launch (dt_reduce_block's
+// rule): each reduces the partials itself, so that the launch that needs dt
+// can also be the one that finds it; workgroup 0 records it.  In two halves,
+// so that the fluxes, which do not need dt, run while the partials come in:
+// load at the start of the kernel, value() (every thread of the NT) where dt
+// is first needed.
+template <int NT>
+struct StepDt {
+  double m = 0., tnow = 0., tmax = 0.;
+  __device__ __forceinline__ StepDt(const DtFold &f, const double *dev) {
+    if (f.npart == 0) {
+      m = dev[0];
+      return;
+    }
+    double p[4] = {0., 0., 0., 0.};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if ((int)threadIdx.x + u * NT < f.npart) p[u] = f.part[threadIdx.x + u * NT];
+    for (int q = threadIdx.x + 4 * NT; q < f.npart; q += NT) p[0] = fmax(p[0], f.part[q]);
+    m = fmax(fmax(p[0], p[1]), fmax(p[2], p[3]));
+    tnow = dev[1];
+    tmax = dev[2];
+  }
+  // a step past t_max, known before dt (step_past_tmax)
+  __device__ __forceinline__ bool past(const DtFold &f) const {
+    if (f.npart == 0) return m == 0.;
+    if (f.use_fixed) return f.fixed_dt == 0.;
+    return tmax >= 0. && !(tnow < tmax);
+  }
+  __device__ __forceinline__ double value(const DtFold &f, double *dev) const {
+    if (f.npart == 0) return m;
+    __shared__ double red[NT / 64];
+    const double mm = wave_max(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mm;
+    __syncthreads();
+    double x = red[0];
+#pragma unroll
+    for (int r = 1; r < NT / 64; ++r) x = fmax(x, red[r]);
+    double dt = f.use_fixed ? f.fixed_dt : f.cour / x;
+    if (!f.use_fixed && tmax >= 0.) {
+      if (!(tnow < tmax))
+        dt = 0.;
+      else if (tnow + dt > tmax)
+        dt = tmax - tnow;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      dev[0] = dt;
+      if (dt != 0.) dev[7] = dt;
+    }
+    return dt;
+  }
+};
+
+// Maximum over a workgroup of NT threads, valid in thread 0.
+template <int NT>
+__device__ __forceinline__ double block_max_nt(double v) {
+  __shared__ double red[NT / 64];
+  v = wave_max(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double m = red[0];
+#pragma unroll
+  for (int q = 1; q < NT / 64; ++q) m = fmax(m, red[q]);
+  return m;
+}
+
+// The value of the lane to the left (right) in a row of 16 lanes (a DPP row);
+// the row's first (last) lane gets its own `end`.  Every lane must be active.
+template <int CTRL>
+__device__ __forceinline__ int dpp_mov(int end, int v) {
+  return __builtin_amdgcn_update_dpp(end, v, CTRL, 0xf, 0xf, false);
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double end, double v) {
+  const int lo = dpp_mov<CTRL>(__double2loint(end), __double2loint(v));
+  const int hi = dpp_mov<CTRL>(__double2hiint(end), __double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float end, float v) {
+  return __int_as_float(dpp_mov<CTRL>(__float_as_int(end), __float_as_int(v)));
+}
+template <int TX, typename T>
+__device__ __forceinline__ T from_left(T v, T end = T(0)) {  // row_shr:1
+  static_assert(TX == 16, "a row of the tile is a DPP row");
+  return dpp_mov<0x111>(end, v);
+}
+template <int TX, typename T>
+__device__ __forceinline__ T from_right(T v, T end = T(0)) {  // row_shl:1
+  static_assert(TX == 16, "a row of the tile is a DPP row");
+  return dpp_mov<0x101>(end, v);
+}
+
+// Value of array a (a uniform address) at byte offset o: with a 32-bit offset
+// the load takes its base from scalar registers and one vector register
+// serves every variable of a cell.
+template <typename T>
+__device__ __forceinline__ T at(const T *a, unsigned o) {
+  return *(const T *)((const char *)a + o);
+}
+template <typename T>
+__device__ __forceinline__ void put(T *a, unsigned o, T v) {
+  *(T *)((char *)a + o) = v;
+}
+
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ double uniform(double v) {
+  const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+  const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+
+// dt over a cell's volume and faces, and the face areas, as the updates form
+// them.  On a uniform grid they are the same for every cell and wait in
+// scalar registers.
+template <bool UG>
+struct ColGeo {
+  double dt, dlx, dly;
+  __device__ __forceinline__ ColGeo(double t, double x, double y, double) : dt(t), dlx(x), dly(y) {}
+  __device__ __forceinline__ double tv(double z) const { return dt / (dlx * dly * z); }
+  __device__ __forceinline__ double tyz(double z) const { return dt / (dly * z); }
+  __device__ __forceinline__ double txz(double z) const { return dt / (dlx * z); }
+  __device__ __forceinline__ double txy() const { return dt / (dlx * dly); }
+  __device__ __forceinline__ double ayz(double z) const { return dly * z; }
+  __device__ __forceinline__ double axz(double z) const { return dlx * z; }
+  __device__ __forceinline__ double axy() const { return dlx * dly; }
+};
+template <>
+struct ColGeo<true> {
+  double v, yz, xz, xy, a_yz, a_xz, a_xy;
+  __device__ __forceinline__ ColGeo(double t, double x, double y, double z)
+      : v(uniform(t / (x * y * z))), yz(uniform(t / (y * z))), xz(uniform(t / (x * z))),
+        xy(uniform(t / (x * y))), a_yz(uniform(y * z)), a_xz(uniform(x * z)),
+        a_xy(uniform(x * y)) {}
+  __device__ __forceinline__ double tv(double) const { return v; }
+  __device__ __forceinline__ double tyz(double) const { return yz; }
+  __device__ __forceinline__ double txz(double) const { return xz; }
+  __device__ __forceinline__ double txy() const { return xy; }
+  __device__ __forceinline__ double ayz(double) const { return a_yz; }
+  __device__ __forceinline__ double axz(double) const { return a_xz; }
+  __device__ __forceinline__ double axy() const { return a_xy; }
+};
+
+// The boundaries of a grid, for the kernels that write the ghost cells along
+// with the active cells they copy (build_ghosts composes per-axis maps, so
+// the ghosts of an active cell are the products of its images per axis).
+struct Bnd {
+  int a1[3], a2[3];  // first and last active index
+  int flag[6];       // BNZ_BC_PERIODIC, _OUTFLOW or _REFLECT per side
+  int ng, dims;
+  int plain;         // no reflecting side
+};
+
+// Images of index x along one axis, bit 0 x itself, bit 1 + g the low ghost
+// a1 - ng + g, bit 1 + ng + g the high ghost a2 + 1 + g.  FACE: the images of
+// a face index of the axis's own normal field (mirrored about the wall face).
+template <bool FACE>
+__device__ __forceinline__ unsigned images(const Bnd &b, int axis, int x) {
+  unsigned m = 1u;
+  if (axis >= b.dims) return m;
+  const int a1 = b.a1[axis], a2 = b.a2[axis], ng = b.ng, n = a2 - a1 + 1;
+  const int lo = b.flag[2 * axis], hi = b.flag[2 * axis + 1];
+  if (lo == BNZ_BC_OUTFLOW) {
+    if (x == a1) m |= ((1u << ng) - 1) << 1;
+  } else {
+    const int q = lo == BNZ_BC_PERIODIC ? x - n : FACE ? 2 * a1 - x : 2 * a1 - 1 - x;
+    if (q >= a1 - ng && q < a1) m |= 1u << (1 + q - (a1 - ng));
+  }
+  if (hi == BNZ_BC_OUTFLOW) {
+    if (x == a2) m |= ((1u << ng) - 1) << (1 + ng);
+  } else {
+    const int q = hi == BNZ_BC_PERIODIC ? x + n : FACE ? 2 * a2 + 2 - x : 2 * a2 + 1 - x;
+    const int q0 = (FACE && hi == BNZ_BC_REFLECT) ? a2 + 2 : a2 + 1;
+    if (q >= q0 && q <= a2 + ng) m |= 1u << (1 + ng + q - (a2 + 1));
+  }
+  return m;
+}
+
+// Index of image bit s of x, and whether that side mirrors it.
+__device__ __forceinline__ int image_at(const Bnd &b, int axis, int s, int x, bool &flip) {
+  flip = false;
+  if (s == 0) return x;
+  const int g = s - 1;
+  flip = b.flag[2 * axis + (g < b.ng ? 0 : 1)] == BNZ_BC_REFLECT;
+  return g < b.ng ? b.a1[axis] - b.ng + g : b.a2[axis] + 1 + (g - b.ng);
+}
+
+// f(cell index, flips) for every combination of images but the cell itself;
+// bit a of flips: mirrored along axis a.
+template <class F>
+__device__ __forceinline__ void each_image(const Bnd &b, const Geo &g, const unsigned m[3], int i,
+                                           int j, int k, const F &f) {
+  for (unsigned mz = m[2]; mz; mz &= mz - 1) {
+    bool fz, fy, fx;
+    const int kk = image_at(b, 2, __builtin_ctz(mz), k, fz);
+    for (unsigned my = m[1]; my; my &= my - 1) {
+      const int jj = image_at(b, 1, __builtin_ctz(my), j, fy);
+      for (unsigned mx = m[0]; mx; mx &= mx - 1) {
+        const int ii = image_at(b, 0, __builtin_ctz(mx), i, fx);
+        if (((mx | my | mz) & 1u) && ii == i && jj == j && kk == k) continue;
+        f(((long)kk * g.nt[1] + jj) * g.nt[0] + ii,
+          (unsigned)fx | ((unsigned)fy << 1) | ((unsigned)fz << 2));
+      }
+    }
+  }
+}
+
+// Whether active cell (i, j, k) has images, or a wall face of its own.
+__device__ __forceinline__ bool near_side(const Bnd &b, int i, int j, int k) {
+  const int x[3] = {i, j, k};
+  bool any = false;
+  for (int a = 0; a < 3; ++a)
+    if (a < b.dims)
+      any = any || x[a] <= b.a1[a] + b.ng || x[a] >= b.a2[a] - b.ng;
+  return any;
+}
+
+// The ghosts of active cell (i, j, k) after its update: cells(dst, flips)
+// copies its cell variables to cell dst, face(a, dst, flip) its face a,
+// wall(a, dst) zeroes face a of dst (the wall face of a reflecting side).
+// Together over the active cells this writes every ghost cell as build_ghosts
+// and the ghost fill do; each target has one source.
+template <class CELLS, class FACE, class WALL>
+__device__ __forceinline__ void scatter_ghosts(const Bnd &b, const Geo &g, int i, int j, int k,
+                                               const CELLS &cells, const FACE &face,
+                                               const WALL &wall) {
+  const unsigned m[3] = {images<false>(b, 0, i), images<false>(b, 1, j), images<false>(b, 2, k)};
+  each_image(b, g, m, i, j, k, cells);
+  const int x[3] = {i, j, k};
+  for (int a = 0; a < 3; ++a) {
+    if (a >= b.dims) {
+      each_image(b, g, m, i, j, k, [&](long dst, unsigned) { face(a, dst, false); });
+      continue;
+    }
+    unsigned f[3] = {m[0], m[1], m[2]};
+    f[a] = a == 0 ? images<true>(b, 0, i) : a == 1 ? images<true>(b, 1, j) : images<true>(b, 2, k);
+    const bool zlo = b.flag[2 * a] == BNZ_BC_REFLECT && x[a] == b.a1[a];
+    const bool zhi = b.flag[2 * a + 1] == BNZ_BC_REFLECT && x[a] == b.a2[a];
+    each_image(b, g, f, i, j, k,
+               [&](long dst, unsigned flips) { face(a, dst, ((flips >> a) & 1u) != 0); });
+    if (zlo || zhi) {
+      // the wall face itself and its images along the other axes
+      unsigned o[3] = {m[0], m[1], m[2]};
+      o[a] = 1u;
+      const long step = a == 0 ? 1 : a == 1 ? g.sy : g.sz;
+      const long self = ((long)k * g.nt[1] + j) * g.nt[0] + i;
+      if (zlo) {
+        wall(a, self);
+        each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst); });
+      }
+      if (zhi) {
+        wall(a, self + step);
+        each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst + step); });
+      }
+    }
+  }
+}
+
+// --------------------------------------------------------------------------
+// Host side
+
+inline Bnd bnd_of(const bnz_ctx *c) {
+  Bnd b;
+  const int lo[3] = {c->i1, c->j1, c->k1}, hi[3] = {c->i2, c->j2, c->k2};
+  for (int a = 0; a < 3; ++a) {
+    b.a1[a] = lo[a];
+    b.a2[a] = hi[a];
+  }
+  for (int q = 0; q < 6; ++q) b.flag[q] = c->p.bc[q];
+  b.ng = c->ng;
+  b.dims = c->dims;
+  b.plain = 1;
+  for (int q = 0; q < 2 * c->dims; ++q)
+    if (b.flag[q] == BNZ_BC_REFLECT) b.plain = 0;
+  return b;
+}
+
+// A launch of tiles with an own range of `span` cells per axis: the tiles'
+// counts and origin.  pred: the whole grid (cells outside the limits are
+// copied); else the cells of flux3_box(L), whose faces a stage solves.
+struct Tiling {
+  int o[2], n[2];
+  int blocks() const { return n[0] * n[1]; }
+};
+inline Tiling tiling2(const bnz_ctx *c, const Lims &L, bool pred, int ex, int ey) {
+  Tiling t;
+  const int e[2] = {ex, ey};
+  for (int a = 0; a < 2; ++a) {
+    const int lo = pred ? 0 : L.lo[a] - 1, hi = pred ? c->nt[a] - 1 : L.hi[a] + 1;
+    t.o[a] = lo;
+    t.n[a] = (hi - lo + e[a]) / e[a];
+  }
+  return t;
+}
+
+// Workgroups of a 3D stage that a CU holds: 256 threads each, compiled for up
+// to 256 registers, with 39 LDS doubles a thread (FP64) or fewer (FP32C).
+// FP32C fits three or four, which measured no faster (256^3: 3.24 ms a step
+// with two, 3.76 with three, 3.27 with four).
+constexpr int STAGE3_PER_CU = 2;
+
+// Cells from which the 3D stages take their workgroups in run_block order
+// (256^3: 4.24 -> 4.17 ms a step; 200x144x168 and below are slower so).
+constexpr long STAGE3_RUN_CELLS = 1L << 23;
+
+// Columns of a 3D stage (stage3_column): tiles in x and y as tiling2, cut in
+// z into runs of nz planes each of which pays two planes of x and y faces
+// more.  The runs are chosen so that the workgroups fill the CUs in as few
+// and as short rounds as possible (STAGE3_PER_CU workgroups per CU and round).
+struct Tiling3 {
+  int o[3], n[3], nz, top;  // origin, tiles per axis, planes per run, last plane
+  int runs;                 // workgroups in run_block order
+  int blocks() const { return n[0] * n[1] * n[2]; }
+};
+inline Tiling3 tiling3(const bnz_ctx *c, const Lims &L, bool pred, bool active, int ex,
+                       int ey) {
+  Tiling3 t;
+  t.runs = c->ncell >= STAGE3_RUN_CELLS;
+  const int e[2] = {ex, ey};
+  const int lo[3] = {c->i1, c->j1, c->k1}, hi[3] = {c->i2, c->j2, c->k2};
+  for (int a = 0; a < 3; ++a) {
+    const int x0 = pred ? 0 : active ? lo[a] : L.lo[a] - 1;
+    const int x1 = pred ? c->nt[a] - 1 : active ? hi[a] : L.hi[a] + 1;
+    t.o[a] = x0;
+    if (a < 2) {
+      t.n[a] = (x1 - x0 + e[a]) / e[a];
+    } else {
+      t.top = x1;
+      const int planes = x1 - x0 + 1;
+      const long cols = (long)t.n[0] * t.n[1], slots = (long)STAGE3_PER_CU * c->ncu;
+      long best = 0;
+      for (int q = 1; q <= planes; ++q) {
+        const int run = (planes + q - 1) / q, runs = (planes + run - 1) / run;
+        const long cost = (cols * runs + slots - 1) / slots * (run + 2);
+        if (!best || cost < best) {
+          best = cost;
+          t.nz = run;
+          t.n[2] = runs;
+        }
+      }
+    }
+  }
+  return t;
+}
+
+// The 3D stages address a variable's plane with 32-bit byte offsets.  Below
+// the lower bounds a column has too few planes to fill the chip, and the
+// separate kernels are faster (us per step, separate -> columns: FP64 64^3
+// 151 -> 155, 128^3 862 -> 732; FP32C 64^3 92 -> 104, 128^3 590 -> 530).
+constexpr long STAGE3_MAX_CELLS = 1L << 29;
+constexpr long STAGE3_MIN_CELLS64 = 400000, STAGE3_MIN_CELLS32 = 1L << 20;
+
+// Grids whose stages run as fused passes: 2D and 3D Van-Leer steps in the
+// default placement (bnz_set_tuning 0, 0, 0).  The upwind EMF, characteristic
+// limiting and user boundaries keep the separate kernels.
+inline bool fused_stages(const bnz_ctx *c) {
+  if (c->dims == 3 && (c->ncell > STAGE3_MAX_CELLS ||
+                       c->ncell < (c->f32 ? STAGE3_MIN_CELLS32 : STAGE3_MIN_CELLS64)))
+    return false;
+  return c->dims >= 2 && !c->p.tintegr && !c->p.ct_upwind && !c->p.char_proj && c->npass == 0 &&
+         c->flux_chunk == 0 && c->emf_chunk == 0 && c->update_chunk == 0;
+}
+
+// Cells up to which a 2D stage takes its small tile (16 x 8: more workgroups
+// on an idle chip; 128^2 20.2 us a step against 23.9 with 16 x 16 tiles),
+// beyond which the big one (32 x 16: fewer rim cells; 32 x 32 is slower, 219
+// against 204 us at 1024^2).
+constexpr long TILE2_SMALL_CELLS = 1L << 16;
+
+// Own cells of the tiles, and the partials their launches can leave.
+constexpr int TILE3[2] = {16, 16};
+constexpr int TILE2_BIG[2] = {32, 16}, TILE2_SMALL[2] = {16, 8};
+inline long tile_parts(const bnz_ctx *c) {
+  const Lims L = integr_lims(c, 0);
+  if (c->dims == 3) return tiling3(c, L, true, false, TILE3[0] - 2, TILE3[1] - 2).blocks();
+  return std::max(tiling2(c, L, true, TILE2_BIG[0] - 2, TILE2_BIG[1] - 2).blocks(),
+                  tiling2(c, L, true, TILE2_SMALL[0] - 2, TILE2_SMALL[1] - 2).blocks());
+}
+
+// A pending dt over more partials than this is reduced by a launch of its
+// own (the first step after an upload of a large grid: k_dt_partial leaves
+// one per 256 cells), not by every workgroup of the stage.
+constexpr int DT_PARTS_IN_STAGE = 4096;
+
+}  // namespace bnz

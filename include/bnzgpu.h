@@ -169,14 +169,19 @@ int bnz_state_size(const bnz_ctx *ctx, long *bytes);
 int bnz_save_state(bnz_ctx *ctx, void *host, long bytes);
 int bnz_load_state(bnz_ctx *ctx, const void *host, long bytes);
 
-/* Work shapes of the 3D Godunov-flux, edge-EMF and stage-update kernels:
-   0 one thread per face/edge/cell in x-fastest order (the default; the
+/* 0, 0, 0 (the default): 2D grids and large 3D grids run each stage of the
+   VL step as one fused pass (fluxes, EMFs and update; characteristic
+   limiting, the upwind EMF and user boundaries excepted).  Any other setting
+   runs the separate kernels.
+   Work shapes of the separate 3D Godunov-flux, edge-EMF and stage-update
+   kernels:
+   0 one thread per face/edge/cell in x-fastest order (the
    flux, EMF and update launches of 3D grids of at least 2^21 cells with
    ghosts then take their workgroups in runs of 16 dealt round-robin over
    the XCDs),
    1 tiles of 64 x 4 cells ordered along z (FP64; FP32C runs it flat),
-   n > 1 slab columns of n rows walked plane by plane.  On 2D FP64 grids emf_chunk
-   places the edge EMFs instead: 0 (the default) forms them inside the
+   n > 1 slab columns of n rows walked plane by plane.  On 2D grids emf_chunk
+   places the edge EMFs of the separate kernels instead: 0 forms them inside the
    update launches up to 2^18 cells with ghosts and in launches of their own
    beyond, 1 always in launches of their own, 2 or more always inside the
    updates.  Results do not depend on either choice.  Chosen by the
