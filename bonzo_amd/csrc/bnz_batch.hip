@@ -19,21 +19,20 @@
 #include <vector>
 
 #include "bnz_batch.hpp"
-#include "bnz_kern64.hpp"
+#include "bnz_tile64.hpp"
 
 using namespace bnz;
 using namespace bnzb;
 
 namespace {
 
-// The hot kernels (flux, EMF, update) are compiled per dimensionality and
-// launched over the work blocks of the boxes of that dimensionality: a 1D
-// box then runs 1D code with the registers 1D code needs.  Their workgroups
-// take the work blocks in run_block order (runs of 16 dealt round-robin over
-// the XCDs, so that an XCD walks neighbouring rows of a box): 2D blasts
-// +3 % (FP64) and +5 % (FP32C) over launch order; the 1D stage kernels keep
-// launch order, which is faster for them.
-template <int ORDER, int RS, int DIMS>
+// The hot kernels are compiled per dimensionality and launched over the work
+// blocks of the boxes of that dimensionality: 1D and 2D boxes run fused
+// stages, 3D boxes separate fluxes, EMFs and updates.  The workgroups of the
+// 2D and 3D kernels take the work blocks in run_block order (runs of 16 dealt
+// round-robin over the XCDs, so that an XCD walks neighbouring rows of a box);
+// the 1D kernels keep launch order, which is faster for them.
+template <int ORDER, int RS>
 __global__ __launch_bounds__(BLK) void kb_flux(const BoxDev *__restrict__ boxes, WList wl,
                                                BoxState st, const double *__restrict__ w,
                                                const double *__restrict__ bf,
@@ -49,12 +48,11 @@ __global__ __launch_bounds__(BLK) void kb_flux(const BoxDev *__restrict__ boxes,
     int i, j, k;
     box_idx(it, t, i, j, k);
     const long o = d.off;
-    flux_cell<ORDER, RS, DIMS>(d.g, w + o, bf + o, fx + o, fy + o, fz + o,
+    flux_cell<ORDER, RS, 3>(d.g, w + o, bf + o, fx + o, fy + o, fz + o,
                                d.L[wl.kt == KF0 ? 0 : 1], i, j, k);
   }
 }
 
-template <int DIMS>
 __global__ __launch_bounds__(BLK) void kb_emf(const BoxDev *__restrict__ boxes, WList wl,
                                               BoxState st, const double *__restrict__ w,
                                               const double *__restrict__ fx,
@@ -71,7 +69,7 @@ __global__ __launch_bounds__(BLK) void kb_emf(const BoxDev *__restrict__ boxes, 
     int i, j, k;
     box_idx(it, t, i, j, k);
     const long o = d.off;
-    emf_edge_d<DIMS>(d.g, w + o, fx + o, fy + o, fz + o, ee + o, i, j, k);
+    emf_edge_d<3>(d.g, w + o, fx + o, fy + o, fz + o, ee + o, i, j, k);
   }
 }
 
@@ -80,7 +78,7 @@ __global__ __launch_bounds__(BLK) void kb_emf(const BoxDev *__restrict__ boxes, 
 // work block).  A finished box is left alone: its faces stay in the buffer
 // its last step wrote, which kb_time_dt tracks (BoxState::fpar) and
 // kb_face_fix makes current when an advance ends.
-template <bool PRED, int DIMS>
+template <bool PRED>
 __global__ __launch_bounds__(BLK) void kb_update(const BoxDev *__restrict__ boxes, WList wl,
                                                  BoxState st, Pools p, int fms_ref) {
   for (int wb = wl.lo + (int)run_block(); wb < wl.hi; wb += gridDim.x) {
@@ -95,15 +93,45 @@ __global__ __launch_bounds__(BLK) void kb_update(const BoxDev *__restrict__ boxe
       int i, j, k;
       box_idx(it, t, i, j, k);
       if (PRED)
-        update_cell_d<DIMS, true, false>(d.g, p.w + o, p.fx + o, p.fy + o, p.fz + o, p.ee + o,
+        update_cell_d<3, true, false>(d.g, p.w + o, p.fx + o, p.fy + o, p.fz + o, p.ee + o,
                                          p.b + o, p.bs + o, p.ws + o, d.L[0], st.dt + b, d.act,
                                          fms_ref, i, j, k);
       else
-        cds = update_cell_d<DIMS, false, true>(d.g, p.w + o, p.fx + o, p.fy + o, p.fz + o,
+        cds = update_cell_d<3, false, true>(d.g, p.w + o, p.fx + o, p.fy + o, p.fz + o,
                                                p.ee + o, p.b + o, p.bs + o, p.w + o, d.L[1],
                                                st.dt + b, d.act, fms_ref, i, j, k);
     }
     if (!PRED) block_max_atomic(cds, st.cmax + b);
+  }
+}
+
+// One stage of the 2D boxes in one pass, a tile per workgroup (stage2_tile).
+// The predictor's faces go to p.ee, the corrector's and their ghosts to p.bs,
+// which the caller makes current.  As in the single grid's 2D stages (k_stage2)
+// no flux goes through HBM, and a step is three launches instead of seven: 24
+// FP32C blasts of side 64 .. 320 to t = 0.1 took 93 ms with separate launches
+// and take 76, the copies to and from the host included.
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+__global__ __launch_bounds__(TX *TY, TX *TY >= 512 ? 4 : 2) void kb_stage2(
+    const BoxDev *__restrict__ boxes, WList wl, BoxState st, Pools p, int fms_ref) {
+  constexpr int NT = TX * TY;
+  __shared__ double lds[tile2_lds<NT>()];
+  for (int wb = wl.lo + (int)run_block(); wb < wl.hi; wb += gridDim.x) {
+    const int b = wl.bmap[wb];
+    if (!st.run[b]) continue;
+    const BoxDev &d = boxes[b];
+    const Box &it = d.items[wl.kt];
+    const int q = wb - d.blk0[wl.kt];
+    const long o = d.off;
+    const double cds = stage2_tile<PRED, ORDER, RS, TX, TY>(
+        d.g, (PRED ? p.w : p.ws) + o, (PRED ? p.b : p.ee) + o, p.w + o, p.b + o,
+        (PRED ? p.ws : p.w) + o, (PRED ? p.ee : p.bs) + o, d.L[PRED ? 0 : 1],
+        [&] { return st.dt[b]; }, d.act, d.bnd, fms_ref, it.lo[0] + q % it.n[0] * (TX - 2),
+        it.lo[1] + q / it.n[0] * (TY - 2), lds);
+    if (!PRED)
+      block_max_atomic<NT>(cds, st.cmax + b);  // ends with a barrier: lds is free again
+    else
+      __syncthreads();
   }
 }
 
@@ -383,38 +411,24 @@ Box mkbox(int i0, int ni, int j0, int nj, int k0, int nk) {
 
 
 
-// fluxes of the 2D and 3D boxes (1D boxes: kb_stage1)
+// fluxes of the 3D boxes
 template <int ORDER, int RS>
 void b_fluxes(bnz_batch *c, const double *w, const double *bf, int kt) {
-  for (int d = 2; d <= 3; ++d) {
-    const WList wl = wlist_dims(c, kt, d);
-    if (wl.hi == wl.lo) continue;
-    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TF]));
-    if (d == 2)
-      hipLaunchKernelGGL((kb_flux<ORDER, RS, 2>), grid, dim3(BLK), 0, c->stream, c->boxes, wl,
-                         c->S, w, bf, c->P.fx, c->P.fy, c->P.fz);
-    else
-      hipLaunchKernelGGL((kb_flux<ORDER, RS, 3>), grid, dim3(BLK), 0, c->stream, c->boxes, wl,
-                         c->S, w, bf, c->P.fx, c->P.fy, c->P.fz);
-  }
+  const WList wl = wlist(c, kt);
+  if (wl.hi == wl.lo) return;
+  hipLaunchKernelGGL((kb_flux<ORDER, RS>), dim3(grid_for(wl.hi - wl.lo, c->cap[TF])), dim3(BLK), 0,
+                     c->stream, c->boxes, wl, c->S, w, bf, c->P.fx, c->P.fy, c->P.fz);
 }
 
-// EMFs of the 2D and 3D boxes (1D boxes form theirs in the update)
+// EMFs of the 3D boxes
 void b_emf(bnz_batch *c, const double *w, int kt) {
-  for (int d = 2; d <= 3; ++d) {
-    const WList wl = wlist_dims(c, kt, d);
-    if (wl.hi == wl.lo) continue;
-    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TE]));
-    if (d == 2)
-      hipLaunchKernelGGL(kb_emf<2>, grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w,
-                         c->P.fx, c->P.fy, c->P.fz, c->P.ee);
-    else
-      hipLaunchKernelGGL(kb_emf<3>, grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w,
-                         c->P.fx, c->P.fy, c->P.fz, c->P.ee);
-  }
+  const WList wl = wlist(c, kt);
+  if (wl.hi == wl.lo) return;
+  hipLaunchKernelGGL(kb_emf, dim3(grid_for(wl.hi - wl.lo, c->cap[TE])), dim3(BLK), 0, c->stream,
+                     c->boxes, wl, c->S, w, c->P.fx, c->P.fy, c->P.fz, c->P.ee);
 }
 
-// stage updates of the 2D and 3D boxes, then the fused stage of the 1D boxes
+// the fused stages of the 1D and of the 2D boxes
 template <bool PRED, int ORDER, int RS>
 void b_stage1(bnz_batch *c) {
   const WList wl = wlist(c, KS1);
@@ -424,29 +438,39 @@ void b_stage1(bnz_batch *c) {
                      c->stream, c->boxes, wl, c->S, c->P, c->p.dt_fms_ref);
 }
 
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+void b_stage2(bnz_batch *c) {
+  const WList wl = wlist(c, PRED ? KP2 : KC2);
+  hipLaunchKernelGGL((kb_stage2<PRED, ORDER, RS, TX, TY>),
+                     dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(TX * TY), 0, c->stream,
+                     c->boxes, wl, c->S, c->P, c->p.dt_fms_ref);
+}
+
+template <bool PRED, int ORDER, int RS>
+void b_stages(bnz_batch *c) {
+  if (c->nblk[PRED ? KP2 : KC2]) {
+    if (c->tile_small) b_stage2<PRED, ORDER, RS, TILE2_SMALL[0], TILE2_SMALL[1]>(c);
+    else b_stage2<PRED, ORDER, RS, TILE2_BIG[0], TILE2_BIG[1]>(c);
+  }
+  b_stage1<PRED, ORDER, RS>(c);
+}
+
+// stage updates of the 3D boxes, then the fused stages of the others
 template <bool PRED>
 void b_update(bnz_batch *c) {
-  const int fr = c->p.dt_fms_ref;
-  for (int d = 2; d <= 3; ++d) {
-    const WList wl = wlist_dims(c, KUPD, d);
-    if (wl.hi == wl.lo) continue;
-    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TU]));
-    if (d == 2)
-      hipLaunchKernelGGL((kb_update<PRED, 2>), grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S,
-                         c->P, fr);
-    else
-      hipLaunchKernelGGL((kb_update<PRED, 3>), grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S,
-                         c->P, fr);
-  }
+  const WList wl = wlist_dims(c, KUPD, 3);
+  if (wl.hi != wl.lo)
+    hipLaunchKernelGGL((kb_update<PRED>), dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(BLK), 0,
+                       c->stream, c->boxes, wl, c->S, c->P, c->p.dt_fms_ref);
   const int order = PRED ? 0 : c->order, rs = c->p.rsolver;
   if (order == 0) {
-    if (rs == BNZ_RS_HLLD) b_stage1<PRED, 0, BNZ_RS_HLLD>(c);
-    else if (rs == BNZ_RS_HLLT) b_stage1<PRED, 0, BNZ_RS_HLLT>(c);
-    else b_stage1<PRED, 0, BNZ_RS_HLL>(c);
+    if (rs == BNZ_RS_HLLD) b_stages<PRED, 0, BNZ_RS_HLLD>(c);
+    else if (rs == BNZ_RS_HLLT) b_stages<PRED, 0, BNZ_RS_HLLT>(c);
+    else b_stages<PRED, 0, BNZ_RS_HLL>(c);
   } else {
-    if (rs == BNZ_RS_HLLD) b_stage1<PRED, 1, BNZ_RS_HLLD>(c);
-    else if (rs == BNZ_RS_HLLT) b_stage1<PRED, 1, BNZ_RS_HLLT>(c);
-    else b_stage1<PRED, 1, BNZ_RS_HLL>(c);
+    if (rs == BNZ_RS_HLLD) b_stages<PRED, 1, BNZ_RS_HLLD>(c);
+    else if (rs == BNZ_RS_HLLT) b_stages<PRED, 1, BNZ_RS_HLLT>(c);
+    else b_stages<PRED, 1, BNZ_RS_HLL>(c);
   }
 }
 
@@ -463,24 +487,24 @@ void b_flux_dispatch(bnz_batch *c, int order, const double *w, const double *bf,
   }
 }
 
-// Ghost fill of every box; with_time: the end-of-step time and dt kernel
-// rides in the last ghost launch (or runs alone if there is none).
+// Ghost fill of every box, or, at the end of a step (with_time), of the boxes
+// whose stages leave their ghosts to it; the end-of-step time and dt kernel
+// then rides in the last ghost launch (or runs alone if there is none).
 void b_ghost(bnz_batch *c, bool with_time) {
-  const int tp = with_time && c->ngops == 0 ? 1 : 0, to = with_time ? 1 : 0;
-  if (c->nghost > 0)
-    hipLaunchKernelGGL(kb_ghost, dim3(grid_for((c->nghost + BLK - 1) / BLK) + tp), dim3(BLK), 0,
-                       c->stream, c->ncell, c->P.w, c->P.b, c->ghost, c->nghost, c->S, c->nbox,
+  const long np = with_time ? c->nghost_step : c->nghost, no = with_time ? c->ngops_step : c->ngops;
+  const int tp = with_time && no == 0 ? 1 : 0, to = with_time ? 1 : 0;
+  if (np > 0)
+    hipLaunchKernelGGL(kb_ghost, dim3(grid_for((np + BLK - 1) / BLK) + tp), dim3(BLK), 0,
+                       c->stream, c->ncell, c->P.w, c->P.b, c->ghost, np, c->S, c->nbox,
                        c->p.cour, tp);
-  if (c->ngops > 0)
-    hipLaunchKernelGGL(kb_ghost_ops, dim3(grid_for((c->ngops + BLK - 1) / BLK) + to), dim3(BLK),
-                       0, c->stream, c->ncell, c->P.w, c->P.b, c->gops, c->ngops, c->S, c->nbox,
+  if (no > 0)
+    hipLaunchKernelGGL(kb_ghost_ops, dim3(grid_for((no + BLK - 1) / BLK) + to), dim3(BLK),
+                       0, c->stream, c->ncell, c->P.w, c->P.b, c->gops, no, c->S, c->nbox,
                        c->p.cour, to);
-  else if (with_time && c->nghost == 0)
+  else if (with_time && np == 0)
     b_time_dt(c);
 }
 
-// One VL step of every running box (vanleer.pyx:94-167): the same launch
-// sequence as the single grid's step.
 // One VL step of every running box; the box dt's were set by the previous
 // step's kb_time_dt (or by init_state's kb_dt).
 template <int ORDER, int RS>
@@ -580,6 +604,8 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   std::vector<size_t> geo_off;  // 12 per box: (dlf, dlfi, icm, icp) x 3 axes
   std::vector<int2> pairs;
   std::vector<GhostOp> gops;
+  std::vector<int2> pairs2;  // of the 2D boxes
+  std::vector<GhostOp> gops2;
   c->hbox.resize(nbox);
   long off = 0;
   for (int b = 0; b < nbox; ++b) {
@@ -642,13 +668,11 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
       if (dims < 2) L.lo[1] = L.hi[1] = 0;
       if (dims < 3) L.lo[2] = L.hi[2] = 0;
       const int il = L.lo[0], iu = L.hi[0], jl = L.lo[1], ju = L.hi[1], kl = L.lo[2], ku = L.hi[2];
-      d.items[o == 0 ? KF0 : KF1] = flux3_box(dims, L);
-      // 1D boxes form their EMFs from the LDS fluxes (EmfLds1D, EmfLds32x1D): no EMF items
+      // 1D and 2D boxes keep their fluxes and EMFs in LDS: no items
+      const Box none = mkbox(0, 0, 0, 0, 0, 0);
+      d.items[o == 0 ? KF0 : KF1] = dims < 3 ? none : flux3_box(dims, L);
       d.items[o == 0 ? KEM0 : KEM1] =
-          dims == 1
-              ? mkbox(0, 0, 0, 0, 0, 0)
-              : mkbox(il, iu + 2 - il, dims >= 2 ? jl : 0, dims >= 2 ? ju + 2 - jl : 1,
-                      dims >= 3 ? kl : 0, dims >= 3 ? ku + 2 - kl : 1);
+          dims < 3 ? none : mkbox(il, iu + 2 - il, jl, ju + 2 - jl, kl, ku + 2 - kl);
     }
     d.items[KUPD] = mkbox(0, nt[0], 0, nt[1], 0, nt[2]);
     d.items[KS1] = dims == 1 ? mkbox(0, nt[0], 0, 1, 0, 1) : mkbox(0, 0, 0, 0, 0, 0);
@@ -659,7 +683,21 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
       d.walls[2 * a] = (a < dims && s.bc[2 * a] == BNZ_BC_REFLECT) ? a1[a] : -1;
       d.walls[2 * a + 1] = (a < dims && s.bc[2 * a + 1] == BNZ_BC_REFLECT) ? a2[a] + 1 : -1;
     }
-    build_ghosts(nt, dims, ng, s.bc, off, pairs, gops);
+    d.bnd.ng = ng;
+    d.bnd.dims = dims;
+    d.bnd.plain = 1;
+    for (int a = 0; a < 3; ++a) {
+      d.bnd.a1[a] = a1[a];
+      d.bnd.a2[a] = a2[a];
+    }
+    for (int q = 0; q < 6; ++q) {
+      d.bnd.flag[q] = s.bc[q];
+      if (q < 2 * dims && s.bc[q] == BNZ_BC_REFLECT) d.bnd.plain = 0;
+    }
+    if (dims == 2)
+      build_ghosts(nt, dims, ng, s.bc, off, pairs2, gops2);
+    else
+      build_ghosts(nt, dims, ng, s.bc, off, pairs, gops);
     off += (long)nt[0] * nt[1] * nt[2];
     if (off >= (1L << 31))
       return bfail(c, BNZ_EINVAL, "batch too large: pool cell indices are 32-bit");
@@ -667,8 +705,28 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   c->ncell = off;
   c->step1 = true;
   for (int b = 0; b < nbox; ++b) c->step1 = c->step1 && c->hbox[b].g.dims == 1;
+  c->nghost_step = (long)pairs.size();
+  c->ngops_step = (long)gops.size();
+  pairs.insert(pairs.end(), pairs2.begin(), pairs2.end());
+  gops.insert(gops.end(), gops2.begin(), gops2.end());
   c->nghost = (long)pairs.size();
   c->ngops = (long)gops.size();
+  // tiles of the 2D boxes, as the single grid's stages (tiling2): together
+  // the boxes fill the chip, so the sum of their cells decides their size
+  long cells2 = 0;
+  bool any[4] = {};
+  for (const BoxDev &d : c->hbox) {
+    any[d.g.dims] = true;
+    if (d.g.dims == 2) cells2 += (long)d.g.nt[0] * d.g.nt[1];
+  }
+  c->tile_small = cells2 <= TILE2_SMALL_CELLS;
+  for (BoxDev &d : c->hbox)
+    for (int o = 0; o < 2; ++o) {
+      const int *e = c->tile_small ? TILE2_SMALL : TILE2_BIG;
+      const Tiling t = tiling2(d.g.nt, d.L[o], o == 0, e[0] - 2, e[1] - 2);
+      d.items[o == 0 ? KP2 : KC2] = d.g.dims == 2 ? mkbox(t.o[0], t.n[0], t.o[1], t.n[1], 0, 1)
+                                                  : mkbox(0, 0, 0, 0, 0, 0);
+    }
   // work blocks: box b owns ceil(items / BLK) consecutive blocks of each
   // list; the 1D boxes come first, then the 2D and the 3D boxes
   std::vector<int> hmap;
@@ -698,12 +756,13 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   struct {
     double **q;
     int rows;
-  } bufs[] = {{&c->P.w, NMODE}, {&c->P.b, 3},          {&c->P.bs, 3},
-              {&c->P.ws, NMODE}, {&c->P.fx, NMODE}, {&c->P.fy, NMODE},
-              {&c->P.fz, NMODE}, {&c->P.ee, 3}};
+  } bufs[] = {{&c->P.w, NMODE}, {&c->P.b, 3},   {&c->P.bs, 3},
+              {&c->P.ws, NMODE}, {&c->P.ee, 3},  {&c->P.fx, NMODE},
+              {&c->P.fy, NMODE}, {&c->P.fz, NMODE}};
   // FP32C keeps prim (upload, download) and the faces in FP64; its work
   // arrays are the FP32 pools below
-  const int nb64 = c->f32 ? 3 : 8;
+  const int nflux = any[1] || any[3] ? 3 : 0;  // the 2D stages have no flux arrays
+  const int nb64 = c->f32 ? 3 : 5 + nflux;
   for (int q = 0; q < nb64; ++q) {
     if (hipMalloc(bufs[q].q, bufs[q].rows * cells * sizeof(double)) != hipSuccess)
       return bfail(c, BNZ_ENOMEM, "device allocation of the box pools failed");
@@ -718,6 +777,7 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
                {&c->Q.bs32, 3}, {&c->Q.fx, 9},  {&c->Q.fy, 9},  {&c->Q.fz, 9},
                {&c->Q.ee, 3}};
     for (auto &q : b32) {
+      if (nflux == 0 && &q >= b32 + 5) break;
       if (hipMalloc(q.q, q.rows * cells * sizeof(float)) != hipSuccess)
         return bfail(c, BNZ_ENOMEM, "device allocation of the FP32 box pools failed");
       BCHK(c, hipMemsetAsync(*q.q, 0, q.rows * cells * sizeof(float), c->stream));

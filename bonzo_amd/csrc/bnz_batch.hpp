@@ -6,20 +6,23 @@
 #include <vector>
 
 #include "bnz_common.hpp"
+#include "bnz_tile.hpp"
 
 namespace bnzb {
 using namespace bnz;
 
 // work lists: fluxes (all directions, one item per cell of the union of the
-// face ranges) and EMFs of the predictor and of the corrector, all cells
-// (stage updates), active cells (init and the first CFL maximum), the cells
-// of the 1D boxes for the fused 1D stage (BLK - 1 per work block) and for
-// the fused 1D step of all-1D FP64 batches (BLK - 5 per work block)
-enum { KF0 = 0, KEM0, KF1, KEM1, KUPD, KACT, KS1, KT1, NK };
+// face ranges) and EMFs of the predictor and of the corrector of the 3D
+// boxes, all cells (3D stage updates, copies), active cells (init and the
+// first CFL maximum), the cells of the 1D boxes for the fused 1D stage (BLK - 1
+// per work block) and for the fused 1D step of all-1D batches (BLK - 5 per
+// work block), the tiles of the 2D boxes for the fused 2D stages (predictor
+// and corrector; a work block is a tile, items are tiles from the origin lo)
+enum { KF0 = 0, KEM0, KF1, KEM1, KUPD, KACT, KS1, KT1, KP2, KC2, NK };
 
-// cells per work block of list kt
+// items per work block of list kt
 __host__ __device__ constexpr int blk_items(int kt) {
-  return kt == KS1 ? BLK - 1 : kt == KT1 ? STEP1_CELLS : BLK;
+  return kt == KS1 ? BLK - 1 : kt == KT1 ? STEP1_CELLS : kt == KP2 || kt == KC2 ? 1 : BLK;
 }
 
 struct BoxDev {
@@ -30,6 +33,7 @@ struct BoxDev {
   Box items[NK];
   int blk0[NK];  // first work block of the box in each list
   int walls[6];  // reflecting wall plane of each side, or -1 (FP32C EMFs)
+  Bnd bnd;       // boundaries (2D stages write the ghosts with the cells)
 };
 
 struct Pools {
@@ -56,15 +60,16 @@ struct BoxState {
 // bits of a non-negative double order like its value).  Every thread of the
 // workgroup calls it (a work block belongs to one box); the closing barrier
 // lets the next work block of a persistent loop reuse red.
+template <int NT = BLK>
 __device__ __forceinline__ void block_max_atomic(double v, unsigned long long *addr) {
-  __shared__ double red[BLK / 64];
+  __shared__ double red[NT / 64];
   v = bnz::wave_max(v);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
     double m = red[0];
 #pragma unroll
-    for (int q = 1; q < BLK / 64; ++q) m = fmax(m, red[q]);
+    for (int q = 1; q < NT / 64; ++q) m = fmax(m, red[q]);
     if (m > 0.) atomicMax(addr, (unsigned long long)__double_as_longlong(m));
   }
   __syncthreads();
@@ -143,6 +148,8 @@ struct bnz_batch {
   int cls[bnzb::NK][4] = {};  // first work block of the 1D, 2D, 3D boxes; nblk
   int cap[bnzb::NTUNE] = {bnzb::PERSIST, bnzb::PERSIST, bnzb::PERSIST};
   long ncell = 0, nghost = 0, ngops = 0;
+  long nghost_step = 0, ngops_step = 0;  // those of the 1D and 3D boxes, which come first
+  bool tile_small = false;               // tile of the 2D stages: small or big
   hipStream_t stream = nullptr;
   bnzb::BoxDev *boxes = nullptr;
   int *bmap = nullptr;

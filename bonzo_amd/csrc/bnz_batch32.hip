@@ -8,7 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bnz_batch.hpp"
-#include "bnz_kern32.hpp"
+#include "bnz_tile32.hpp"
 
 using namespace bnz;
 using namespace bnzb;
@@ -22,9 +22,8 @@ __device__ __forceinline__ Walls box_walls(const BoxDev &d) {
   return wl;
 }
 
-// The flux, EMF and update kernels are compiled per dimensionality and
-// launched over the work blocks of the boxes of that dimensionality.
-template <int ORDER, int RS, typename BF, int DIMS>
+// The flux, EMF and update kernels of the 3D boxes.
+template <int ORDER, int RS, typename BF>
 __global__ __launch_bounds__(BLK) void kb32_flux(const BoxDev *__restrict__ boxes, WList wl,
                                                  BoxState st, const float *__restrict__ w,
                                                  const BF *__restrict__ bf,
@@ -41,13 +40,12 @@ __global__ __launch_bounds__(BLK) void kb32_flux(const BoxDev *__restrict__ boxe
     int i, j, k;
     box_idx(it, t, i, j, k);
     const long o = d.off;
-    flux32_cell<ORDER, RS, BF, DIMS>(d.g, w + o, bf + o, fx + o, fy + o, fz + o,
+    flux32_cell<ORDER, RS, BF, 3>(d.g, w + o, bf + o, fx + o, fy + o, fz + o,
                                      d.L[wl.kt == KF0 ? 0 : 1], i, j, k, ng);
   }
   if (ng) atomicAdd(nguard, ng);
 }
 
-template <int DIMS>
 __global__ __launch_bounds__(BLK) void kb32_emf(const BoxDev *__restrict__ boxes, WList wl,
                                                 BoxState st, const float *__restrict__ w,
                                                 const float *__restrict__ fx,
@@ -64,14 +62,14 @@ __global__ __launch_bounds__(BLK) void kb32_emf(const BoxDev *__restrict__ boxes
     int i, j, k;
     box_idx(it, t, i, j, k);
     const long o = d.off;
-    emf32_edge<DIMS>(d.g, w + o, fx + o, fy + o, fz + o, ee + o, box_walls(d), i, j, k);
+    emf32_edge<3>(d.g, w + o, fx + o, fy + o, fz + o, ee + o, box_walls(d), i, j, k);
   }
 }
 
 // Stage update of every cell of the running boxes (update32_pred /
 // update32_corr); the corrector folds the CFL maximum into the box's cmax.
 // A finished box is left alone (its faces: BoxState::fpar, kb_face_fix).
-template <bool PRED, int DIMS>
+template <bool PRED>
 __global__ __launch_bounds__(BLK) void kb32_update(const BoxDev *__restrict__ boxes, WList wl,
                                                    BoxState st, Pools P, Pools32 Q,
                                                    int fms_ref) {
@@ -89,15 +87,51 @@ __global__ __launch_bounds__(BLK) void kb32_update(const BoxDev *__restrict__ bo
       if (PRED) {
         const Pred32 a{Q.w32 + o, Q.uh + o, P.b + o, Q.fx + o, Q.fy + o,
                        Q.fz + o,  Q.ee + o, Q.bs32 + o, Q.ws32 + o};
-        update32_pred<DIMS>(d.g, a, d.L[0], st.dt + b, i, j, k);
+        update32_pred<3>(d.g, a, d.L[0], st.dt + b, i, j, k);
       } else {
         const Corr32 a{Q.uh + o, Q.ul + o, P.b + o, Q.fx + o, Q.fy + o,
                        Q.fz + o, Q.ee + o, P.bs + o, Q.w32 + o};
-        cds = update32_corr<DIMS>(d.g, a, d.L[1], st.dt + b, d.act, fms_ref, i, j, k);
+        cds = update32_corr<3>(d.g, a, d.L[1], st.dt + b, d.act, fms_ref, i, j, k);
       }
     }
     if (!PRED) block_max_atomic(cds, st.cmax + b);
   }
+}
+
+// One FP32C stage of the 2D boxes in one pass (stage2_tile32), as the FP64
+// kb_stage2; the predictor's faces go to Q.bs32.
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+__global__ __launch_bounds__(TX *TY, TX *TY >= 512 ? 4 : 2) void kb32_stage2(
+    const BoxDev *__restrict__ boxes, WList wl, BoxState st, Pools P, Pools32 Q, int fms_ref,
+    int *nguard) {
+  constexpr int NT = TX * TY;
+  using BF = typename std::conditional<PRED, double, float>::type;
+  __shared__ float lds[tile2_lds32<NT>()];
+  int ng = 0;
+  for (int wb = wl.lo + (int)run_block(); wb < wl.hi; wb += gridDim.x) {
+    const int b = wl.bmap[wb];
+    if (!st.run[b]) continue;
+    const BoxDev &d = boxes[b];
+    const Box &it = d.items[wl.kt];
+    const int q = wb - d.blk0[wl.kt];
+    const long o = d.off;
+    const Pred32 ap{Q.w32 + o, Q.uh + o, P.b + o, nullptr, nullptr, nullptr, nullptr, Q.bs32 + o,
+                    Q.ws32 + o};
+    const Corr32 ac{Q.uh + o, Q.ul + o, P.b + o, nullptr, nullptr, nullptr, nullptr, P.bs + o,
+                    Q.w32 + o};
+    const BF *bf;
+    if constexpr (PRED) bf = P.b + o;
+    else bf = Q.bs32 + o;
+    const double cds = stage2_tile32<PRED, ORDER, RS, TX, TY>(
+        d.g, (PRED ? Q.w32 : Q.ws32) + o, bf, ap, ac, d.L[PRED ? 0 : 1],
+        [&] { return st.dt[b]; }, d.act, d.bnd, box_walls(d), fms_ref,
+        it.lo[0] + q % it.n[0] * (TX - 2), it.lo[1] + q / it.n[0] * (TY - 2), lds, ng);
+    if (!PRED)
+      block_max_atomic<NT>(cds, st.cmax + b);  // ends with a barrier: lds is free again
+    else
+      __syncthreads();
+  }
+  if (ng) atomicAdd(nguard, ng);
 }
 
 // One FP32C stage of the 1D boxes in one pass (stage32_cell), as the FP64
@@ -300,20 +334,14 @@ __global__ __launch_bounds__(BLK) void kb32_ghost_ops(Ghost32 p, const GhostOp *
     ghost32_op(p, ops[t]);
 }
 
-// fluxes of the 2D and 3D boxes (1D boxes: kb32_stage1)
+// fluxes of the 3D boxes
 template <int ORDER, int RS, typename BF>
 void flux_launch(bnz_batch *c, const float *w, const BF *bf, int kt) {
-  for (int d = 2; d <= 3; ++d) {
-    const WList wl = wlist_dims(c, kt, d);
-    if (wl.hi == wl.lo) continue;
-    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TF]));
-    if (d == 2)
-      hipLaunchKernelGGL((kb32_flux<ORDER, RS, BF, 2>), grid, dim3(BLK), 0, c->stream, c->boxes,
-                         wl, c->S, w, bf, c->Q.fx, c->Q.fy, c->Q.fz, c->nguard);
-    else
-      hipLaunchKernelGGL((kb32_flux<ORDER, RS, BF, 3>), grid, dim3(BLK), 0, c->stream, c->boxes,
-                         wl, c->S, w, bf, c->Q.fx, c->Q.fy, c->Q.fz, c->nguard);
-  }
+  const WList wl = wlist(c, kt);
+  if (wl.hi == wl.lo) return;
+  hipLaunchKernelGGL((kb32_flux<ORDER, RS, BF>), dim3(grid_for(wl.hi - wl.lo, c->cap[TF])),
+                     dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w, bf, c->Q.fx, c->Q.fy,
+                     c->Q.fz, c->nguard);
 }
 
 template <typename BF>
@@ -328,21 +356,15 @@ void fluxes(bnz_batch *c, int order, const float *w, const BF *bf, int kt) {
   }
 }
 
-// EMFs of the 2D and 3D boxes (1D boxes form theirs in the update)
+// EMFs of the 3D boxes
 void emfs(bnz_batch *c, const float *w, int kt) {
-  for (int d = 2; d <= 3; ++d) {
-    const WList wl = wlist_dims(c, kt, d);
-    if (wl.hi == wl.lo) continue;
-    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TE]));
-    if (d == 2)
-      hipLaunchKernelGGL(kb32_emf<2>, grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w,
-                         c->Q.fx, c->Q.fy, c->Q.fz, c->Q.ee);
-    else
-      hipLaunchKernelGGL(kb32_emf<3>, grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w,
-                         c->Q.fx, c->Q.fy, c->Q.fz, c->Q.ee);
-  }
+  const WList wl = wlist(c, kt);
+  if (wl.hi == wl.lo) return;
+  hipLaunchKernelGGL(kb32_emf, dim3(grid_for(wl.hi - wl.lo, c->cap[TE])), dim3(BLK), 0, c->stream,
+                     c->boxes, wl, c->S, w, c->Q.fx, c->Q.fy, c->Q.fz, c->Q.ee);
 }
 
+// the fused stages of the 1D and of the 2D boxes
 template <bool PRED, int ORDER, int RS>
 void stage1(bnz_batch *c) {
   const WList wl = wlist(c, KS1);
@@ -352,28 +374,37 @@ void stage1(bnz_batch *c) {
                      c->stream, c->boxes, wl, c->S, c->P, c->Q, c->p.dt_fms_ref, c->nguard);
 }
 
-// stage updates of the 2D and 3D boxes, then the fused stage of the 1D boxes
+template <bool PRED, int ORDER, int RS, int TX, int TY>
+void stage2(bnz_batch *c) {
+  const WList wl = wlist(c, PRED ? KP2 : KC2);
+  hipLaunchKernelGGL((kb32_stage2<PRED, ORDER, RS, TX, TY>),
+                     dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(TX * TY), 0, c->stream,
+                     c->boxes, wl, c->S, c->P, c->Q, c->p.dt_fms_ref, c->nguard);
+}
+
+template <bool PRED, int ORDER, int RS>
+void stages(bnz_batch *c) {
+  if (c->nblk[PRED ? KP2 : KC2]) {
+    if (c->tile_small) stage2<PRED, ORDER, RS, TILE2_SMALL[0], TILE2_SMALL[1]>(c);
+    else stage2<PRED, ORDER, RS, TILE2_BIG[0], TILE2_BIG[1]>(c);
+  }
+  stage1<PRED, ORDER, RS>(c);
+}
+
+// stage updates of the 3D boxes, then the fused stages of the others
 template <bool PRED>
 void updates(bnz_batch *c) {
-  const int fr = c->p.dt_fms_ref;
-  for (int d = 2; d <= 3; ++d) {
-    const WList wl = wlist_dims(c, KUPD, d);
-    if (wl.hi == wl.lo) continue;
-    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TU]));
-    if (d == 2)
-      hipLaunchKernelGGL((kb32_update<PRED, 2>), grid, dim3(BLK), 0, c->stream, c->boxes, wl,
-                         c->S, c->P, c->Q, fr);
-    else
-      hipLaunchKernelGGL((kb32_update<PRED, 3>), grid, dim3(BLK), 0, c->stream, c->boxes, wl,
-                         c->S, c->P, c->Q, fr);
-  }
-  const int order = PRED ? 0 : c->order;
-  if (order == 0) {
-    if (c->p.rsolver == BNZ_RS_HLLD) stage1<PRED, 0, BNZ_RS_HLLD>(c);
-    else stage1<PRED, 0, BNZ_RS_HLL>(c);
+  const WList wl = wlist_dims(c, KUPD, 3);
+  if (wl.hi != wl.lo)
+    hipLaunchKernelGGL((kb32_update<PRED>), dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(BLK),
+                       0, c->stream, c->boxes, wl, c->S, c->P, c->Q, c->p.dt_fms_ref);
+  const bool hlld = c->p.rsolver == BNZ_RS_HLLD;
+  if (PRED || c->order == 0) {
+    if (hlld) stages<PRED, 0, BNZ_RS_HLLD>(c);
+    else stages<PRED, 0, BNZ_RS_HLL>(c);
   } else {
-    if (c->p.rsolver == BNZ_RS_HLLD) stage1<PRED, 1, BNZ_RS_HLLD>(c);
-    else stage1<PRED, 1, BNZ_RS_HLL>(c);
+    if (hlld) stages<PRED, 1, BNZ_RS_HLLD>(c);
+    else stages<PRED, 1, BNZ_RS_HLL>(c);
   }
 }
 
@@ -425,15 +456,17 @@ void b32_step(bnz_batch *c) {
   }
   std::swap(c->P.b, c->P.bs);
   const Ghost32 p = ghost_arrays(c);
-  // the end-of-step time and dt kernel rides in the last ghost launch
-  const int tp = c->ngops == 0 ? 1 : 0;
-  if (c->nghost > 0)
-    hipLaunchKernelGGL(kb32_ghost, dim3(grid_for((c->nghost + BLK - 1) / BLK) + tp), dim3(BLK),
-                       0, c->stream, p, c->ghost, c->nghost, c->S, c->nbox, c->p.cour, tp);
-  if (c->ngops > 0)
-    hipLaunchKernelGGL(kb32_ghost_ops, dim3(grid_for((c->ngops + BLK - 1) / BLK) + 1), dim3(BLK),
-                       0, c->stream, p, c->gops, c->ngops, c->S, c->nbox, c->p.cour, 1);
-  else if (c->nghost == 0)
+  // the ghosts the stages left; the end-of-step time and dt kernel rides in
+  // the last ghost launch
+  const long np = c->nghost_step, no = c->ngops_step;
+  const int tp = no == 0 ? 1 : 0;
+  if (np > 0)
+    hipLaunchKernelGGL(kb32_ghost, dim3(grid_for((np + BLK - 1) / BLK) + tp), dim3(BLK),
+                       0, c->stream, p, c->ghost, np, c->S, c->nbox, c->p.cour, tp);
+  if (no > 0)
+    hipLaunchKernelGGL(kb32_ghost_ops, dim3(grid_for((no + BLK - 1) / BLK) + 1), dim3(BLK),
+                       0, c->stream, p, c->gops, no, c->S, c->nbox, c->p.cour, 1);
+  else if (np == 0)
     b_time_dt(c);
 }
 

@@ -452,7 +452,7 @@ void stage32(bnz_ctx *c, int order, const Lims &L) {
 // bs32 -> uh, ul, w32 in place and the faces to bs.
 template <bool PRED, int ORDER, int RS, int TX, int TY>
 void stage2_launch32(bnz_ctx *c, const Lims &L) {
-  const Tiling tl = tiling2(c, L, PRED, TX - 2, TY - 2);
+  const Tiling tl = tiling2(c->nt, L, PRED, TX - 2, TY - 2);
   const DtFold dtf = PRED ? take_dt(c) : DtFold{};
   const Pred32 ap{c->w32, c->uh, c->b, c->fx32, c->fy32, c->fz32, c->ee32, c->bs32, c->ws32};
   const Corr32 ac{c->uh, c->ul, c->b, c->fx32, c->fy32, c->fz32, c->ee32, c->bs, c->w32};

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(TX *TY, STAGE3_PER_CU) void k_stage3(Geo g, const d
 // caller swaps with b; no EMF array is needed here).
 template <bool PRED, int ORDER, int RS, int TX, int TY>
 void stage2_launch(bnz_ctx *c, const Lims &L) {
-  const Tiling tl = tiling2(c, L, PRED, TX - 2, TY - 2);
+  const Tiling tl = tiling2(c->nt, L, PRED, TX - 2, TY - 2);
   const DtFold dtf = PRED ? take_dt(c) : DtFold{};
   Launch t(c, PRED ? "stage_pred" : "stage_corr");
   hipLaunchKernelGGL((k_stage2<PRED, ORDER, RS, TX, TY>), dim3(tl.blocks()), dim3(TX * TY), 0,

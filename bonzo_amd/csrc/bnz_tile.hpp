@@ -291,11 +291,11 @@ struct Tiling {
   int o[2], n[2];
   int blocks() const { return n[0] * n[1]; }
 };
-inline Tiling tiling2(const bnz_ctx *c, const Lims &L, bool pred, int ex, int ey) {
+inline Tiling tiling2(const int *nt, const Lims &L, bool pred, int ex, int ey) {
   Tiling t;
   const int e[2] = {ex, ey};
   for (int a = 0; a < 2; ++a) {
-    const int lo = pred ? 0 : L.lo[a] - 1, hi = pred ? c->nt[a] - 1 : L.hi[a] + 1;
+    const int lo = pred ? 0 : L.lo[a] - 1, hi = pred ? nt[a] - 1 : L.hi[a] + 1;
     t.o[a] = lo;
     t.n[a] = (hi - lo + e[a]) / e[a];
   }
@@ -382,8 +382,8 @@ constexpr int TILE2_BIG[2] = {32, 16}, TILE2_SMALL[2] = {16, 8};
 inline long tile_parts(const bnz_ctx *c) {
   const Lims L = integr_lims(c, 0);
   if (c->dims == 3) return tiling3(c, L, true, false, TILE3[0] - 2, TILE3[1] - 2).blocks();
-  return std::max(tiling2(c, L, true, TILE2_BIG[0] - 2, TILE2_BIG[1] - 2).blocks(),
-                  tiling2(c, L, true, TILE2_SMALL[0] - 2, TILE2_SMALL[1] - 2).blocks());
+  return std::max(tiling2(c->nt, L, true, TILE2_BIG[0] - 2, TILE2_BIG[1] - 2).blocks(),
+                  tiling2(c->nt, L, true, TILE2_SMALL[0] - 2, TILE2_SMALL[1] - 2).blocks());
 }
 
 // A pending dt over more partials than this is reduced by a launch of its
