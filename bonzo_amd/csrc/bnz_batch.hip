@@ -555,6 +555,14 @@ int blaunch_check(bnz_batch *c) {
   return BNZ_OK;
 }
 
+// A box's arrays in the pools; a null host array is left out.
+int box_segs(bnz_batch *c, const BoxDev &d, double *prim, double *bfld, size_t n, Seg *s) {
+  int k = 0;
+  if (prim) s[k++] = Seg{c->P.w + d.off, prim, c->ncell, NMODE, (long)n};
+  if (bfld) s[k++] = Seg{c->P.b + d.off, bfld, c->ncell, 3, (long)n};
+  return k;
+}
+
 void drop_graph(bnz_batch *c) {
   if (c->exec) (void)hipGraphExecDestroy(c->exec);
   if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -871,13 +879,9 @@ int bnz_batch_upload(bnz_batch *c, int box, const double *prim, const double *bf
   if (!c->stream) return bfail(c, BNZ_ESTATE, "batch was not created");
   const BoxDev &d = c->hbox[box];
   const size_t n = (size_t)d.g.nt[0] * d.g.nt[1] * d.g.nt[2];
-  for (int v = 0; v < NMODE && prim; ++v)
-    BCHK(c, hipMemcpyAsync(c->P.w + v * c->ncell + d.off, prim + v * n, n * sizeof(double),
-                           hipMemcpyHostToDevice, c->stream));
-  for (int v = 0; v < 3 && bfld; ++v)
-    BCHK(c, hipMemcpyAsync(c->P.b + v * c->ncell + d.off, bfld + v * n, n * sizeof(double),
-                           hipMemcpyHostToDevice, c->stream));
-  BCHK(c, hipStreamSynchronize(c->stream));
+  Seg seg[2];
+  const int k = box_segs(c, d, const_cast<double *>(prim), const_cast<double *>(bfld), n, seg);
+  BCHK(c, c->link.up(c->p.device, c->stream, seg, k));
   c->ready = false;
   c->w_stale = false;
   return BNZ_OK;
@@ -893,15 +897,12 @@ int bnz_batch_download(bnz_batch *c, int box, double *prim, double *bfld) {
     if (rc) return rc;
     c->w_stale = false;
   }
-  BCHK(c, hipStreamSynchronize(c->stream));
   const BoxDev &d = c->hbox[box];
   const size_t n = (size_t)d.g.nt[0] * d.g.nt[1] * d.g.nt[2];
-  for (int v = 0; v < NMODE && prim; ++v)
-    BCHK(c, hipMemcpy(prim + v * n, c->P.w + v * c->ncell + d.off, n * sizeof(double),
-                      hipMemcpyDeviceToHost));
-  for (int v = 0; v < 3 && bfld; ++v)
-    BCHK(c, hipMemcpy(bfld + v * n, c->P.b + v * c->ncell + d.off, n * sizeof(double),
-                      hipMemcpyDeviceToHost));
+  Seg seg[2];
+  const int k = box_segs(c, d, prim, bfld, n, seg);
+  if (!k) BCHK(c, hipStreamSynchronize(c->stream));
+  BCHK(c, c->link.down(c->p.device, c->stream, seg, k));
   return BNZ_OK;
 }
 

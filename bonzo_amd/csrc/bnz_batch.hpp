@@ -170,6 +170,7 @@ struct bnz_batch {
   int *hrun = nullptr;         // pinned host copies of the running-box count (2 slots)
   hipEvent_t ev[2] = {nullptr, nullptr};
   bool ready = false;
+  bnz::HostLink link;  // uploads and downloads
   std::string err;
 };
 

@@ -12,6 +12,7 @@
 
 #include "../../include/bnzgpu.h"
 #include "bnz_phys.hpp"
+#include "bnz_xfer.hpp"
 
 namespace bnz {
 
@@ -422,6 +423,7 @@ struct bnz_ctx {
   double *hbuf = nullptr;
   hipEvent_t hev[2] = {nullptr, nullptr};
   std::vector<KTime> ktimes;
+  bnz::HostLink link;  // uploads and downloads
   std::string err;
 };
 

@@ -922,25 +922,27 @@ int bnz_get_shape(const bnz_ctx *c, int *ntot3, int *ng) {
   return BNZ_OK;
 }
 
+// The prim and face arrays; a null host array is left out.
+static int state_segs(bnz_ctx *c, double *prim, double *bfld, Seg *s) {
+  int k = 0;
+  if (prim) s[k++] = Seg{c->w, prim, NMODE * c->ncell, 1, NMODE * c->ncell};
+  if (bfld) s[k++] = Seg{c->b, bfld, 3 * c->ncell, 1, 3 * c->ncell};
+  return k;
+}
+
 int bnz_upload(bnz_ctx *c, const double *prim, const double *bfld) {
   if (!c || !c->stream) return BNZ_EINVAL;
   c->dt_parts = 0;
   c->pdt_pending = false;
-  // ordered after the steps still running on the context's stream (a plain
-  // hipMemcpy would not wait for a non-blocking stream)
   if (c->p.hydro && bfld)  // the hydro build has no field
     for (long q = 0; q < 3 * c->ncell; ++q)
       if (bfld[q] != 0.)
         return fail(c, BNZ_EINVAL, "hydro build: every face field value must be zero");
-  if (prim)
-    HIPCHK(c, hipMemcpyAsync(c->w, prim, NMODE * c->ncell * sizeof(double),
-                             hipMemcpyHostToDevice, c->stream));
-  if (bfld)
-    HIPCHK(c, hipMemcpyAsync(c->b, bfld, 3 * c->ncell * sizeof(double), hipMemcpyHostToDevice,
-                             c->stream));
-  else if (c->p.hydro)
+  Seg seg[2];
+  const int k = state_segs(c, const_cast<double *>(prim), const_cast<double *>(bfld), seg);
+  HIPCHK(c, c->link.up(c->p.device, c->stream, seg, k));
+  if (!bfld && c->p.hydro)
     HIPCHK(c, hipMemsetAsync(c->b, 0, 3 * c->ncell * sizeof(double), c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   // the uploaded state has no ghosts, cell-centred field or FP32C words yet
   c->ready = false;
   return BNZ_OK;
@@ -952,9 +954,10 @@ int bnz_download(bnz_ctx *c, double *prim, double *bfld, double *cons) {
     int rc = f32_to64(c);
     if (rc) return rc;
   }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (prim) HIPCHK(c, hipMemcpy(prim, c->w, NMODE * c->ncell * sizeof(double), hipMemcpyDeviceToHost));
-  if (bfld) HIPCHK(c, hipMemcpy(bfld, c->b, 3 * c->ncell * sizeof(double), hipMemcpyDeviceToHost));
+  Seg seg[2];
+  const int k = state_segs(c, prim, bfld, seg);
+  if (!k) HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, c->link.down(c->p.device, c->stream, seg, k));
   if (cons) {
     // ws is dead between steps; it holds prim2cons(prim) for the copy (the
     // FP32 step has no FP64 ws, so a temporary is used)
@@ -964,9 +967,9 @@ int bnz_download(bnz_ctx *c, double *prim, double *bfld, double *cons) {
                        c->w, tmp);
     int rc = check_launch(c);
     if (!rc) {
-      hipError_t e1 = hipStreamSynchronize(c->stream);
-      hipError_t e2 = hipMemcpy(cons, tmp, NMODE * c->ncell * sizeof(double), hipMemcpyDeviceToHost);
-      if (e1 != hipSuccess || e2 != hipSuccess) rc = fail(c, BNZ_EHIP, "copy of cons failed");
+      const Seg s{tmp, cons, NMODE * c->ncell, 1, NMODE * c->ncell};
+      if (c->link.down(c->p.device, c->stream, &s, 1) != hipSuccess)
+        rc = fail(c, BNZ_EHIP, "copy of cons failed");
     }
     if (tmp != c->ws) (void)hipFree(tmp);
     if (rc) return rc;
