@@ -20,6 +20,7 @@
 
 #include "bnz_batch.hpp"
 #include "bnz_tile64.hpp"
+#include "bnz_tube64.hpp"
 
 using namespace bnz;
 using namespace bnzb;
@@ -178,6 +179,46 @@ __global__ __launch_bounds__(BLK) void kb_step1(const BoxDev *__restrict__ boxes
                                               sw);
     block_max_atomic(cds, st.cmax + b);  // ends with a barrier: sf, sw are free again
   }
+}
+
+// Up to nsteps steps of each box of a batch of short 1D boxes, a workgroup per
+// box (tube_run), so that no box waits on another; the longest go first.
+// Beside longer boxes this is not done: their steps take as long either way
+// (256 tubes of 64 to 1024 cells, the short ones so on a stream of their own:
+// 26.1 ms for 27.1, and 3 ms to make the stream).
+// ms to t = 0.1, launches of single steps -> this: 256 tubes of 48 to 250 cells
+// 5.0 -> 1.6, 256 of 64 to 500 10.4 -> 4.9, 384 of those 12.2 -> 5.7.
+template <int ORDER, int RS, int NT>
+__global__ __launch_bounds__(NT) void kb_tubes(const BoxDev *__restrict__ boxes,
+                                               const int *__restrict__ tubes, BoxState st, Pools p,
+                                               int fms_ref, double cour, int nsteps) {
+  __shared__ double lds[TUBE_SLOTS * NT];
+  const int b = tubes[blockIdx.x];
+  const BoxDev &d = boxes[b];
+  const long o = d.off;
+  TubeClock ck{st.t[b], st.tmax[b], 0., st.dt[b], cour, true};
+  double last = 0.;
+  const int taken = tube_run<ORDER, RS, NT>(d.g, d.bnd, p.w + o, p.b + o, p.fx + o, fms_ref, nsteps,
+                                            false, ck, last, lds);
+  if (threadIdx.x == 0 && taken) {
+    st.t[b] = ck.t;
+    st.steps[b] += taken;
+    if (ck.t < ck.tmax) st.dt[b] = ck.dt;
+  }
+}
+
+// The boxes still short of t_max, as time_dt_block counts them.
+__global__ __launch_bounds__(BLK) void kb_tubes_left(int nbox, BoxState st) {
+  __shared__ int cnt;
+  if (threadIdx.x == 0) cnt = 0;
+  __syncthreads();
+  for (int b = threadIdx.x; b < nbox; b += BLK) {
+    const int on = st.t[b] < st.tmax[b] ? 1 : 0;
+    st.run[b] = on;
+    if (on) atomicAdd(&cnt, 1);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *st.nrun = cnt;
 }
 
 // CFL maximum of the current prim over the active cells (after init).
@@ -514,6 +555,33 @@ void b_step1(bnz_batch *c) {
                      0, c->stream, c->boxes, wl, c->S, c->P, c->p.dt_fms_ref);
 }
 
+template <int ORDER, int RS>
+void tubes_launch(bnz_batch *c, int nsteps) {
+#define TUBES(NT)                                                                               \
+  hipLaunchKernelGGL((kb_tubes<ORDER, RS, NT>), dim3(c->nbox), dim3(tube_threads(c->tube_nt)),  \
+                     0, c->stream, c->boxes, c->tubes, c->S, c->P, c->p.dt_fms_ref, c->p.cour,  \
+                     nsteps)
+  switch (tube_class(c->tube_nt)) {
+    case 0: TUBES(TUBE_NT[0]); break;
+    default: TUBES(TUBE_NT[1]);
+  }
+#undef TUBES
+}
+
+// Up to nsteps steps of every box.
+void b_tubes(bnz_batch *c, int nsteps) {
+  const int rs = c->p.rsolver;
+  if (c->order == 0) {
+    if (rs == BNZ_RS_HLLD) tubes_launch<0, BNZ_RS_HLLD>(c, nsteps);
+    else if (rs == BNZ_RS_HLLT) tubes_launch<0, BNZ_RS_HLLT>(c, nsteps);
+    else tubes_launch<0, BNZ_RS_HLL>(c, nsteps);
+  } else {
+    if (rs == BNZ_RS_HLLD) tubes_launch<1, BNZ_RS_HLLD>(c, nsteps);
+    else if (rs == BNZ_RS_HLLT) tubes_launch<1, BNZ_RS_HLLT>(c, nsteps);
+    else tubes_launch<1, BNZ_RS_HLL>(c, nsteps);
+  }
+}
+
 void b_step(bnz_batch *c) {
   if (c->f32) {
     b32_step(c);  // ends with the ghost fill and the time kernel
@@ -569,6 +637,60 @@ void drop_graph(bnz_batch *c) {
   c->exec = nullptr;
   c->graph = nullptr;
   c->graph_b = nullptr;
+}
+
+// Steps until every box has reached its t_max, or max_steps; n: the steps
+// launched.
+int advance_steps(bnz_batch *c, int max_steps, int use_graph, int &n) {
+  if (use_graph && c->exec && c->graph_b != c->P.b) drop_graph(c);
+  if (use_graph && !c->exec) {
+    c->graph_b = c->P.b;
+    BCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+    b_step(c);
+    b_step(c);  // two swaps: the face buffers are back where capture began
+    hipGraph_t g = nullptr;
+    const hipError_t e = hipStreamEndCapture(c->stream, &g);
+    if (e != hipSuccess) {
+      c->graph_b = nullptr;
+      return bfail(c, BNZ_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+    }
+    c->graph = g;
+    BCHK(c, hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0));
+  }
+  // Steps go out in chunks (REPLAYS graph replays, or one eager step), each
+  // followed by a copy of the running-box count into a pinned slot.  The
+  // host reads a chunk's count while the next chunk runs, so the device does
+  // not drain between chunks; a chunk issued after the last box finished only
+  // launches idle kernels.
+  constexpr int REPLAYS = 4;
+  auto chunk = [&](int slot) -> int {
+    if (use_graph) {
+      for (int r = 0; r < REPLAYS && (max_steps <= 0 || n < max_steps); ++r) {
+        BCHK(c, hipGraphLaunch(c->exec, c->stream));
+        n += 2;
+      }
+    } else {
+      b_step(c);
+      n += 1;
+    }
+    int rc = blaunch_check(c);
+    if (rc) return rc;
+    BCHK(c, hipMemcpyAsync(c->hrun + slot, c->S.nrun, sizeof(int), hipMemcpyDeviceToHost,
+                           c->stream));
+    BCHK(c, hipEventRecord(c->ev[slot], c->stream));
+    return BNZ_OK;
+  };
+  int slot = 0;
+  int rc = chunk(slot);
+  if (rc) return rc;
+  for (;;) {
+    const bool more = max_steps <= 0 || n < max_steps;
+    if (more && (rc = chunk(slot ^ 1)) != 0) return rc;
+    BCHK(c, hipEventSynchronize(c->ev[slot]));
+    if (c->hrun[slot] == 0 || !more) break;
+    slot ^= 1;
+  }
+  return BNZ_OK;
 }
 
 }  // namespace
@@ -825,6 +947,17 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   // box scalars: dt, t, tmax, cmax (8 bytes each), run, steps, fpar (4 bytes),
   // nrun
   const size_t nb = nbox;
+  int longest = 0;
+  for (const BoxDev &d : c->hbox) longest = std::max(longest, d.g.nt[0]);
+  if (c->step1 && !c->f32 && longest <= TUBE_CELLS) {
+    c->tube_nt = longest;
+    std::vector<int> h(nb);
+    for (int b = 0; b < nbox; ++b) h[b] = b;
+    std::stable_sort(h.begin(), h.end(),
+                     [&](int x, int y) { return c->hbox[x].g.nt[0] > c->hbox[y].g.nt[0]; });
+    BCHK(c, hipMalloc(&c->tubes, nb * sizeof(int)));
+    BCHK(c, hipMemcpy(c->tubes, h.data(), nb * sizeof(int), hipMemcpyHostToDevice));
+  }
   const size_t words = 4 * nb + (3 * nb + 1 + 1) / 2;
   BCHK(c, hipMalloc(&c->sbuf, words * sizeof(double)));
   c->S.dt = c->sbuf;
@@ -857,6 +990,7 @@ int bnz_batch_destroy(bnz_batch *c) {
   if (c->nguard) (void)hipFree(c->nguard);
   if (c->boxes) (void)hipFree(c->boxes);
   if (c->bmap) (void)hipFree(c->bmap);
+  if (c->tubes) (void)hipFree(c->tubes);
   if (c->ghost) (void)hipFree(c->ghost);
   if (c->gops) (void)hipFree(c->gops);
   for (hipEvent_t e : c->ev)
@@ -938,55 +1072,24 @@ int bnz_batch_init_state(bnz_batch *c) {
 int bnz_batch_advance(bnz_batch *c, int max_steps, int use_graph, int *nsteps) {
   if (!c) return BNZ_EINVAL;
   if (!c->ready) return bfail(c, BNZ_ESTATE, "bnz_batch_init_state has not run");
-  if (use_graph && c->exec && c->graph_b != c->P.b) drop_graph(c);
-  if (use_graph && !c->exec) {
-    c->graph_b = c->P.b;
-    BCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    b_step(c);
-    b_step(c);  // two swaps: the face buffers are back where capture began
-    hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(c->stream, &g);
-    if (e != hipSuccess) {
-      c->graph_b = nullptr;
-      return bfail(c, BNZ_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-    }
-    c->graph = g;
-    BCHK(c, hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0));
-  }
-  // Steps go out in chunks (REPLAYS graph replays, or one eager step), each
-  // followed by a copy of the running-box count into a pinned slot.  The
-  // host reads a chunk's count while the next chunk runs, so the device does
-  // not drain between chunks; a chunk issued after the last box finished only
-  // launches idle kernels.
-  constexpr int REPLAYS = 4;
   int n = 0;
-  auto chunk = [&](int slot) -> int {
-    if (use_graph) {
-      for (int r = 0; r < REPLAYS && (max_steps <= 0 || n < max_steps); ++r) {
-        BCHK(c, hipGraphLaunch(c->exec, c->stream));
-        n += 2;
-      }
-    } else {
-      b_step(c);
-      n += 1;
-    }
-    int rc = blaunch_check(c);
-    if (rc) return rc;
-    BCHK(c, hipMemcpyAsync(c->hrun + slot, c->S.nrun, sizeof(int), hipMemcpyDeviceToHost,
-                           c->stream));
-    BCHK(c, hipEventRecord(c->ev[slot], c->stream));
+  if (c->tube_nt) {
+    // TUBE_STEPS a launch (graph or not; with graphs an odd limit is rounded up)
+    const int most = max_steps <= 0 || !use_graph ? max_steps : (max_steps + 1) / 2 * 2;
+    do {
+      const int q = most <= 0 ? TUBE_STEPS : std::min(TUBE_STEPS, most - n);
+      b_tubes(c, q);
+      n += q;
+      hipLaunchKernelGGL(kb_tubes_left, dim3(1), dim3(BLK), 0, c->stream, c->nbox, c->S);
+      if (const int rc = blaunch_check(c)) return rc;
+      BCHK(c, hipMemcpyAsync(c->hrun, c->S.nrun, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+      BCHK(c, hipStreamSynchronize(c->stream));
+    } while (c->hrun[0] && (most <= 0 || n < most));
+    if (nsteps) *nsteps = n;
     return BNZ_OK;
-  };
-  int slot = 0;
-  int rc = chunk(slot);
-  if (rc) return rc;
-  for (;;) {
-    const bool more = max_steps <= 0 || n < max_steps;
-    if (more && (rc = chunk(slot ^ 1)) != 0) return rc;
-    BCHK(c, hipEventSynchronize(c->ev[slot]));
-    if (c->hrun[slot] == 0 || !more) break;
-    slot ^= 1;
   }
+  int rc = advance_steps(c, max_steps, use_graph, n);
+  if (rc) return rc;
   // faces of the boxes that finished an odd number of steps ago
   hipLaunchKernelGGL(kb_face_fix, dim3(grid_for(c->nblk[KUPD])), dim3(BLK), 0, c->stream,
                      c->boxes, wlist(c, KUPD), c->S, c->P.b, c->P.bs,

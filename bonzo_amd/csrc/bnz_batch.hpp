@@ -158,6 +158,8 @@ struct bnz_batch {
   bnz::GhostOp *gops = nullptr;
   bnzb::Pools P{};
   bool f32 = false;
+  int tube_nt = 0;       // every box a short 1D one in FP64: cells of the largest
+  int *tubes = nullptr;  // then the boxes, the largest first
   bool step1 = false;  // all boxes 1D: fused steps, state buffers swap like the faces
   bnzb::Pools32 Q{};
   int *nguard = nullptr;  // guarded FP32 HLLD faces

@@ -718,5 +718,6 @@ void launch_ghost64(bnz_ctx *c);
 void launch_ghost_step64(bnz_ctx *c);  // a step's fill: also t += dt, step += 1
 // the FP64 step compiled with contraction (bnz_gpu64f.hip)
 void fma_step_body(bnz_ctx *c);
+void fma_tube(bnz_ctx *c, int nsteps);
 
 }  // namespace bnz

@@ -470,6 +470,22 @@ void any_step(bnz_ctx *c) {
   else launch_step_body(c);
 }
 
+// n steps, each with its CFL dt.
+void any_steps(bnz_ctx *c, int n) {
+  if (tube_grid(c)) {
+    for (; n > 0; n -= TUBE_STEPS) {
+      launch_dt(c, 0, 0.);
+      if (c->p.precision == BNZ_PREC_FP64_FMA) fma_tube(c, std::min(n, TUBE_STEPS));
+      else launch_tube(c, std::min(n, TUBE_STEPS));
+    }
+    return;
+  }
+  for (int s = 0; s < n; ++s) {
+    any_dt(c, 0, 0.);
+    any_step(c);
+  }
+}
+
 // Validation, shape, index ranges and coordinates of a grid (the host part
 // of BnzGrid/BnzIntegr construction); no device work.
 int configure_grid(bnz_ctx *c, const bnz_params *p) {
@@ -1036,10 +1052,7 @@ int bnz_run_steps(bnz_ctx *c, int nsteps) {
   if (!c->ready) return fail(c, BNZ_ESTATE, "bnz_init_state has not run");
   const double nomax = -1.;
   HIPCHK(c, hipMemcpyAsync(c->dev + 2, &nomax, sizeof(double), hipMemcpyHostToDevice, c->stream));
-  for (int s = 0; s < nsteps; ++s) {
-    any_dt(c, 0, 0.);
-    any_step(c);
-  }
+  any_steps(c, nsteps);
   return check_launch(c);
 }
 
@@ -1061,14 +1074,16 @@ int bnz_advance(bnz_ctx *c, double tmax, int max_steps, int *nsteps) {
     // replayed: its launches carry only device pointers and sizes, and the
     // buffers it swaps are back in place after its even number of steps.
     // Right after an upload, a state load or a change of work shapes the
-    // first chunk runs eagerly.
-    constexpr int CHUNK = 8;
+    // first chunk runs eagerly.  A short 1D grid's chunk is one launch, which
+    // ends at t_max by itself (tube_run).
+    const bool tube = tube_grid(c);
+    const int CHUNK = tube ? TUBE_STEPS : 8;
     int launched = 0;
     auto chunk = [&](int slot) -> int {
       const bool full = max_steps <= 0 || launched + CHUNK <= max_steps;
       const bnz_ctx::ChunkKey key = chunk_key(c);
       const bool replay = c->gexec && key == c->gkey;
-      if (c->step_graph && full && !c->timing &&
+      if (c->step_graph && !tube && full && !c->timing &&
           (replay || (c->has_steady && key == c->steady))) {
         if (!replay) drop_chunk_graph(c);
         if (!c->gexec) {
@@ -1095,11 +1110,9 @@ int bnz_advance(bnz_ctx *c, double tmax, int max_steps, int *nsteps) {
           c->has_steady = false;
         }
       } else {
-        int r = 0;
-        for (; r < CHUNK && (max_steps <= 0 || launched < max_steps); ++r, ++launched) {
-          any_dt(c, 0, 0.);
-          any_step(c);
-        }
+        const int r = max_steps <= 0 ? CHUNK : std::min(CHUNK, max_steps - launched);
+        any_steps(c, r);
+        launched += r;
         if (r == CHUNK && chunk_key(c) == key) {
           c->steady = key;
           c->has_steady = true;

@@ -14,5 +14,6 @@
 namespace bnz {
 
 void fma_step_body(bnz_ctx *c) { launch_step_body(c); }
+void fma_tube(bnz_ctx *c, int nsteps) { launch_tube(c, nsteps); }
 
 }  // namespace bnz

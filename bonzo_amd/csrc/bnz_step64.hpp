@@ -9,7 +9,8 @@
 //   predictor: flux3, emf, update<pred>        (donor cell, dt/2)
 //   corrector: flux3, emf, update<corr>        (PLM, dt; CFL maximum fused)
 //   ghost (+ ghost_ops for reflecting sides), time_advance
-// 1D grids run the whole step as one fused pass (k_step1).
+// 1D grids run the whole step as one fused pass (k_step1), short ones many
+// steps in one launch (k_tube).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -18,6 +19,7 @@
 #include "bnz_kern64.hpp"
 #include "bnz_rk3.hpp"
 #include "bnz_tile64.hpp"
+#include "bnz_tube64.hpp"
 
 namespace {
 
@@ -248,6 +250,39 @@ __global__ __launch_bounds__(TX *TY, STAGE3_PER_CU) void k_stage3(Geo g, const d
   if (!PRED) {
     const double m = block_max_nt<NT>(cds);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
+  }
+}
+
+// Up to nsteps steps of a short 1D grid (tube_run) by one workgroup.  Starts
+// from the CFL partials of dtf, leaves one, and keeps dev as the launches of
+// the single steps would.
+template <int ORDER, int RS, int NT>
+__global__ __launch_bounds__(NT) void k_tube(Geo g, Bnd bnd, double *w, double *b,
+                                             const double *__restrict__ fx_old, int fms_ref,
+                                             int nsteps, double *dev, DtFold dtf, double *part) {
+  __shared__ double lds[TUBE_SLOTS * NT];
+  __shared__ double red0[NT / 64];
+  const int i = threadIdx.x;
+  double m = 0.;
+  for (int q = i; q < dtf.npart; q += blockDim.x) m = fmax(m, dtf.part[q]);
+  m = wave_max(m);
+  if ((i & 63) == 0) red0[i >> 6] = m;
+  __syncthreads();
+  m = red0[0];
+  for (int q = 1; q < (int)blockDim.x / 64; ++q) m = fmax(m, red0[q]);
+  TubeClock ck{dev[1], dev[2], m, 0., dtf.cour, dev[2] >= 0.};
+  ck.next_dt();
+  double last = 0.;
+  const int taken = tube_run<ORDER, RS, NT>(g, bnd, w, b, fx_old, fms_ref, nsteps, true, ck, last,
+                                            lds);
+  if (i == 0) {
+    part[0] = ck.m;
+    dev[0] = taken < nsteps ? 0. : last;
+    if (taken) {
+      dev[1] = ck.t;
+      dev[3] += (double)taken;
+      dev[7] = last;
+    }
   }
 }
 
@@ -503,6 +538,39 @@ void launch_rk3_body(bnz_ctx *c) {
 }
 
 // One VL step after the dt kernels (vanleer.pyx:100-163).
+template <int ORDER, int RS>
+void tube_launch(bnz_ctx *c, int nsteps) {
+  const DtFold dtf = take_dt(c);
+  Launch t(c, "tube");
+#define TUBE(NT)                                                                                 \
+  hipLaunchKernelGGL((k_tube<ORDER, RS, NT>), dim3(1), dim3(tube_threads(c->nt[0])), 0,          \
+                     c->stream, c->g, bnd_of(c), c->w, c->b, c->fx, cfl_mode(c), nsteps, c->dev, \
+                     dtf, c->part)
+  switch (tube_class(c->nt[0])) {
+    case 0: TUBE(TUBE_NT[0]); break;
+    default: TUBE(TUBE_NT[1]);
+  }
+#undef TUBE
+  c->dt_parts = 1;
+}
+
+// Up to nsteps steps of a grid that tube_grid admits, the first one's dt
+// deferred (launch_dt).
+void launch_tube(bnz_ctx *c, int nsteps) {
+  const int rs = rs_kern(c);
+#define TUBE(RS)                                          \
+  do {                                                    \
+    if (c->order) tube_launch<1, RS>(c, nsteps);          \
+    else tube_launch<0, RS>(c, nsteps);                   \
+  } while (0)
+  if (rs == BNZ_RS_HLLD) TUBE(BNZ_RS_HLLD);
+  else if (rs == BNZ_RS_HLLT) TUBE(BNZ_RS_HLLT);
+  else if (rs == BNZ_RS_HLLC) TUBE(BNZ_RS_HLLC);
+  else if (rs == RS_HLL_HYDRO) TUBE(RS_HLL_HYDRO);
+  else TUBE(BNZ_RS_HLL);
+#undef TUBE
+}
+
 void launch_step_body(bnz_ctx *c) {
   if (c->p.tintegr) {
     launch_rk3_body(c);

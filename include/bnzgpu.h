@@ -318,8 +318,10 @@ int bnz_batch_init_state(bnz_batch *b);
    are then launched in pairs).  Steps go out in chunks (four pairs, or one
    eager step) and the host reads a chunk's count of running boxes while
    the next chunk runs, so up to one chunk may run after the last box
-   finished (a box at its t_max idles).  *nsteps gets the number of step
-   launches; bnz_batch_get_times gives the steps each box took. */
+   finished (a box at its t_max idles).  An FP64 batch of 1D boxes of at most
+   512 cells each, ghosts included, runs up to 256 steps a launch, and a box
+   ends at its t_max by itself.  *nsteps gets the number of step
+   launches (there 256 for each); bnz_batch_get_times gives the steps each box took. */
 int bnz_batch_advance(bnz_batch *b, int max_steps, int use_graph, int *nsteps);
 /* Workgroups of the stage launches: at most flux_blocks (2D/3D fluxes),
    emf_blocks (EMFs) and update_blocks (2D/3D updates and the fused 1D
