@@ -15,7 +15,7 @@ using namespace bnz;
 // face ranges) and EMFs of the predictor and of the corrector of the 3D
 // boxes, all cells (3D stage updates, copies), active cells (init and the
 // first CFL maximum), the cells of the 1D boxes for the fused 1D stage (BLK - 1
-// per work block) and for the fused 1D step of all-1D batches (BLK - 5 per
+// per work block) and for the fused 1D step of all-1D batches (BLK - 6 per
 // work block), the tiles of the 2D boxes for the fused 2D stages (predictor
 // and corrector; a work block is a tile, items are tiles from the origin lo)
 enum { KF0 = 0, KEM0, KF1, KEM1, KUPD, KACT, KS1, KT1, KP2, KC2, NK };
@@ -54,6 +54,7 @@ struct BoxState {
   int *nrun;                 // boxes still short of t_max after the last step
   int *fpar;                 // steps a finished box sat out, mod 2: its faces are
                              // in the other face buffer when 1
+  int *ticket;               // work blocks of the box that ended a fused 1D step
 };
 
 // Maximum of v over the workgroup folded into *addr with one atomic (the

@@ -18,9 +18,9 @@ namespace bnz {
 
 constexpr int NVAR_STATE = 9;
 constexpr int BLK = 256;
-// cells a workgroup owns in a fused 1D step (step1_block): the predictor
-// also computes 2 cells below and 3 above them
-constexpr int STEP1_CELLS = BLK - 5;
+// cells a workgroup owns in a fused 1D step (step1_block): it also stands on
+// the 3 cells beside them on either side
+constexpr int STEP1_CELLS = BLK - 6;
 
 // --------------------------------------------------------------------------
 // Geometry passed by value to every kernel.
@@ -395,6 +395,8 @@ struct bnz_ctx {
   double *dev = nullptr;      // dt, t, tmax, step
   double *part = nullptr;     // CFL partials (the last corrector's, kept for the next dt)
   long npart_cap = 0;
+  double *part2 = nullptr;    // 1D: the partials alternate with part (step1_folds)
+  int *ticket = nullptr;      // 1D: workgroups of the step that have ended
   double *rpart = nullptr;    // partials of the diag and history reductions
   std::vector<double> h_dlf[3], h_dlfi[3], h_icm[3], h_icp[3], h_dlv[3];
   bnz::Geo g{};
@@ -712,6 +714,11 @@ inline DtFold take_dt(bnz_ctx *c) {
   if (c->pdt_pending) f = c->pdt;
   c->pdt_pending = false;
   return f;
+}
+// 1D FP64 VL grids whose step is one launch (k_step1): all without user
+// boundaries.
+inline bool step1_folds(const bnz_ctx *c) {
+  return c->dims == 1 && !c->f32 && !c->p.tintegr && c->npass == 0;
 }
 void flush_dt(bnz_ctx *c);
 void launch_ghost64(bnz_ctx *c);

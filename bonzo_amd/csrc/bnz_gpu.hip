@@ -462,9 +462,9 @@ void any_dt(bnz_ctx *c, int use_fixed, double fixed_dt) {
   else launch_dt(c, use_fixed, fixed_dt);
 }
 void any_step(bnz_ctx *c) {
-  // 1D VL steps and RK3 steps read dt in their first launch; 2D and 3D VL
-  // steps reduce it in their first flux launch
-  if (c->dims == 1 || c->p.tintegr) flush_dt(c);
+  // VL steps reduce dt in their first launch, but for 1D ones in FP32C or with
+  // user boundaries, and RK3 steps, which read it there
+  if ((c->dims == 1 && !step1_folds(c)) || c->p.tintegr) flush_dt(c);
   if (c->f32) f32_step_body(c);
   else if (c->p.precision == BNZ_PREC_FP64_FMA) fma_step_body(c);
   else launch_step_body(c);
@@ -899,6 +899,10 @@ int bnz_create(const bnz_params *p, bnz_ctx **out) {
                              (long)(c->nt[0] + STEP1_CELLS - 1) / STEP1_CELLS});
   }
   HIPCHK(c, hipMalloc(&c->part, c->npart_cap * sizeof(double)));
+  if (c->dims == 1) {
+    HIPCHK(c, hipMalloc(&c->part2, c->npart_cap * sizeof(double)));
+    c->ticket = (int *)(c->dev + 5);
+  }
   // diag and history reduce into their own buffer, so the CFL partials the
   // last corrector left stay valid and the next dt does not depend on them
   HIPCHK(c, hipMalloc(&c->rpart, (size_t)blocks_for(a.total()) * std::max(NDIAG, NHIST) *
@@ -914,7 +918,7 @@ int bnz_destroy(bnz_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   collect_timing(c);
   double *bufs[] = {c->w,   c->ws,  c->b,    c->bs,  c->fx,  c->fy, c->fz, c->ee,
-                    c->geo, c->dev, c->part, c->rpart, c->uc, c->uss, c->bss};
+                    c->geo, c->dev, c->part, c->part2, c->rpart, c->uc, c->uss, c->bss};
   for (double *q : bufs)
     if (q) (void)hipFree(q);
   drop_chunk_graph(c);

@@ -70,28 +70,52 @@ __global__ __launch_bounds__(BLK) void k_flux3(Geo g, const double *__restrict__
 // the cells from b * STEP1_CELLS; the new prim and faces go to wout and
 // bout, which the host then swaps with w and b; the workgroup's CFL maximum
 // goes to part.
-template <int ORDER, int RS, bool CP = false>
+//   FOLD: the launch is the whole step.  It reduces its dt from the CFL
+// partials of dtf (workgroup 0 records it), writes the ghosts with the cells,
+// and its last workgroup advances the time (ticket, 0 between launches), which
+// by then every workgroup has read; the partials go to another buffer than
+// dtf's.  As three launches (dt, step, ghosts) a step of 512 cells took 12.7 us
+// and takes 10.4 (FMA 11.8, 9.7), some 5 of them from launch to launch; with
+// every phase of step1_block loading what it needs 11.4.
+template <int ORDER, int RS, bool CP = false, bool FOLD = false>
 __global__ __launch_bounds__(BLK) void k_step1(Geo g, const double *__restrict__ w,
                                                const double *__restrict__ bf,
                                                double *__restrict__ wout,
                                                double *__restrict__ bout,
-                                               const double *__restrict__ fx_old, Lims L0,
-                                               Lims L1, const double *__restrict__ dts, Box act,
-                                               int fms_ref, double *__restrict__ part) {
-  __shared__ double sf[NMODE * BLK];
-  __shared__ double sw[NMODE * BLK];
+                                               const double *__restrict__ fx_old,
+                                               double *dev, int fms_ref,
+                                               DtFold dtf, Bnd bnd, int *ticket,
+                                               double *__restrict__ part) {
+  __shared__ double lds[TUBE_SLOTS * BLK];
   const int i0 = blockIdx.x * STEP1_CELLS;
-  if (dts[0] == 0.) {  // a step past t_max: the state is carried into the new buffers
+  const double t0 = FOLD ? dev[1] : 0.;
+  const StepDt<BLK> sd(dtf, dev);  // (no FOLD: no fold, dev[0])
+  double dt = 0., cds = -1.;
+  if (!sd.past(dtf))
+    cds = step1_block<ORDER, RS, CP>(g, w, bf, wout, bout, fx_old, bnd, FOLD,
+                                     [&] { return dt = sd.value(dtf, dev); }, true, fms_ref, i0,
+                                     lds);
+  if (dt == 0.) {  // a step past t_max: the state is carried into the new buffers
+    if (FOLD && blockIdx.x == 0 && threadIdx.x == 0) dev[0] = 0.;
     const int i = i0 + threadIdx.x;
     if (threadIdx.x < STEP1_CELLS && i < g.nt[0]) {
       for (int n = 0; n < NMODE; ++n) wout[n * g.sv + i] = w[n * g.sv + i];
       for (int a = 0; a < 3; ++a) bout[a * g.sv + i] = bf[a * g.sv + i];
     }
-    return;
+    if (!FOLD) return;
+    // and the partials
+    cds = 0.;
+    for (int q = blockIdx.x * BLK + threadIdx.x; q < dtf.npart; q += gridDim.x * BLK)
+      cds = fmax(cds, dtf.part[q]);
   }
-  const double cds = step1_block<ORDER, RS, CP>(g, w, bf, wout, bout, fx_old, L0, L1, dts, act,
-                                                fms_ref, i0, sf, sw);
   block_max_to(cds, part);
+  if (FOLD && threadIdx.x == 0 && dt != 0.) {
+    if (atomicAdd(ticket, 1) == (int)gridDim.x - 1) {
+      *ticket = 0;
+      dev[1] = t0 + dt;
+      dev[3] += 1.;
+    }
+  }
 }
 
 // --------------------------------------------------------------------------
@@ -458,35 +482,42 @@ void launch_update(bnz_ctx *c, bool pred, const Lims &L, const double *we = null
 
 // A 1D step as one fused launch (k_step1): w, b -> ws, bs, then swapped.
 template <int ORDER, int RS>
-void step1_launch(bnz_ctx *c, const Lims &L0, const Lims &L1) {
+void step1_launch(bnz_ctx *c) {
   const int nb = (c->nt[0] + STEP1_CELLS - 1) / STEP1_CELLS;
+  const bool fold = step1_folds(c);
+  const DtFold dtf = fold ? take_dt(c) : DtFold{};
   Launch t(c, "step1");
-  if (ORDER == 1 && c->p.char_proj)
-    hipLaunchKernelGGL((k_step1<ORDER, RS, true>), dim3(nb), dim3(BLK), 0, c->stream, c->g, c->w,
-                       c->b, c->ws, c->bs, c->fx, L0, L1, c->dev, active_box(c),
-                       cfl_mode(c), c->part);
-  else
-    hipLaunchKernelGGL((k_step1<ORDER, RS, false>), dim3(nb), dim3(BLK), 0, c->stream, c->g, c->w,
-                       c->b, c->ws, c->bs, c->fx, L0, L1, c->dev, active_box(c),
-                       cfl_mode(c), c->part);
+#define STEP1(CP, FOLD)                                                                         \
+  hipLaunchKernelGGL((k_step1<ORDER, RS, CP, FOLD>), dim3(nb), dim3(BLK), 0, c->stream, c->g,   \
+                     c->w, c->b, c->ws, c->bs, c->fx, c->dev, cfl_mode(c), dtf,                 \
+                     bnd_of(c), c->ticket, fold ? c->part2 : c->part)
+  if (ORDER == 1 && c->p.char_proj) {
+    if (fold) STEP1(true, true);
+    else STEP1(true, false);
+  } else {
+    if (fold) STEP1(false, true);
+    else STEP1(false, false);
+  }
+#undef STEP1
+  if (fold) std::swap(c->part, c->part2);
   c->dt_parts = nb;
   std::swap(c->w, c->ws);  // the faces swap with the other stages' below
 }
 
-void launch_step1(bnz_ctx *c, const Lims &L0, const Lims &L1) {
+void launch_step1(bnz_ctx *c) {
   const int rs = rs_kern(c);
   if (c->order == 0) {
-    if (rs == BNZ_RS_HLLD) step1_launch<0, BNZ_RS_HLLD>(c, L0, L1);
-    else if (rs == BNZ_RS_HLLT) step1_launch<0, BNZ_RS_HLLT>(c, L0, L1);
-    else if (rs == BNZ_RS_HLLC) step1_launch<0, BNZ_RS_HLLC>(c, L0, L1);
-    else if (rs == RS_HLL_HYDRO) step1_launch<0, RS_HLL_HYDRO>(c, L0, L1);
-    else step1_launch<0, BNZ_RS_HLL>(c, L0, L1);
+    if (rs == BNZ_RS_HLLD) step1_launch<0, BNZ_RS_HLLD>(c);
+    else if (rs == BNZ_RS_HLLT) step1_launch<0, BNZ_RS_HLLT>(c);
+    else if (rs == BNZ_RS_HLLC) step1_launch<0, BNZ_RS_HLLC>(c);
+    else if (rs == RS_HLL_HYDRO) step1_launch<0, RS_HLL_HYDRO>(c);
+    else step1_launch<0, BNZ_RS_HLL>(c);
   } else {
-    if (rs == BNZ_RS_HLLD) step1_launch<1, BNZ_RS_HLLD>(c, L0, L1);
-    else if (rs == BNZ_RS_HLLT) step1_launch<1, BNZ_RS_HLLT>(c, L0, L1);
-    else if (rs == BNZ_RS_HLLC) step1_launch<1, BNZ_RS_HLLC>(c, L0, L1);
-    else if (rs == RS_HLL_HYDRO) step1_launch<1, RS_HLL_HYDRO>(c, L0, L1);
-    else step1_launch<1, BNZ_RS_HLL>(c, L0, L1);
+    if (rs == BNZ_RS_HLLD) step1_launch<1, BNZ_RS_HLLD>(c);
+    else if (rs == BNZ_RS_HLLT) step1_launch<1, BNZ_RS_HLLT>(c);
+    else if (rs == BNZ_RS_HLLC) step1_launch<1, BNZ_RS_HLLC>(c);
+    else if (rs == RS_HLL_HYDRO) step1_launch<1, RS_HLL_HYDRO>(c);
+    else step1_launch<1, BNZ_RS_HLL>(c);
   }
 }
 
@@ -588,7 +619,7 @@ void launch_step_body(bnz_ctx *c) {
     return;
   }
   if (c->dims == 1) {  // the whole step through LDS
-    launch_step1(c, L0, L1);
+    launch_step1(c);
   } else {
     // predictor: donor cell, dt/2, lims of order 0; ws and bs are new buffers
     launch_flux_dispatch(c, 0, c->w, c->b, L0);
@@ -603,7 +634,7 @@ void launch_step_body(bnz_ctx *c) {
     launch_update(c, false, L1, fly ? c->ws : nullptr);
   }
   std::swap(c->b, c->bs);
-  launch_ghost_step64(c);  // and the time advance
+  if (!step1_folds(c)) launch_ghost_step64(c);  // and the time advance
 }
 
 }  // namespace

@@ -118,3 +118,41 @@ def test_batch_tubes_pieces_match_one_run():
     assert np.array_equal(ta[0], tb[0]) and np.array_equal(ta[1], tb[1])
     for x, y in zip(da, db):
         assert np.array_equal(x[0], y[0]) and np.array_equal(x[1], y[1])
+
+
+@pytest.mark.parametrize("precision,char_proj", [("fp64", False), ("fp64", True),
+                                                 ("fp64fma", False)])
+@pytest.mark.parametrize("nx", [508, 747, 748, 2503])
+def test_one_launch_steps_against_the_oracle(nx, precision, char_proj):
+    """Steps of one launch at the sizes where its workgroups end (251 cells
+    each), every boundary: IEEE bit for bit, FMA to 1e-12 relative L1."""
+    from bonzo_amd._lib import Context
+    from oracle.oracle import OracleSim
+    bc = SIDES[nx % 5]
+    print(f"case: {nx} {precision} char {char_proj} bc {bc}", flush=True)
+    s, prim, bfld = _state(nx, 1, 1, 3, 120 + nx)
+    bfld[0][:] = 0.0 if 2 in bc else 0.3
+    o = OracleSim(nx, bc=bc, char_proj=char_proj)
+    o.prim[:] = prim
+    o.bfld[:] = bfld
+    o.init()
+    o.advance_steps(9)
+    g = Context(nx, bc=bc, precision=precision, char_proj=char_proj)
+    for graph in (False, True):
+        g.set_step_graph(graph)
+        g.upload(prim, bfld)
+        g.init_state()
+        assert g.advance(1e9, 9) == 9
+        gp, gb = g.download()
+        for x, y in ((gp, o.prim), (gb, o.bfld)):
+            x, y = x[..., 3:-3], y[..., 3:-3]
+            if precision == "fp64":
+                assert np.array_equal(x, y)
+            else:
+                for v in range(x.shape[0]):
+                    den = max(np.abs(y[v]).sum(), 1e-9 * np.abs(prim[0]).sum())
+                    assert np.abs(x[v] - y[v]).sum() <= 1e-12 * den, v
+        t, n, dt = g.time()
+        assert g.advance(t + 0.4 * dt) == 1 and g.time()[0] == t + 0.4 * dt
+    g.close()
+    o.close()
