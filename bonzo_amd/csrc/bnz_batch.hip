@@ -113,7 +113,7 @@ __global__ __launch_bounds__(BLK) void kb_update(const BoxDev *__restrict__ boxe
 // FP32C blasts of side 64 .. 320 to t = 0.1 took 93 ms with separate launches
 // and take 76, the copies to and from the host included.
 template <bool PRED, int ORDER, int RS, int TX, int TY>
-__global__ __launch_bounds__(TX *TY, TX *TY >= 512 ? 4 : 2) void kb_stage2(
+__global__ __launch_bounds__(TX *TY, 2) void kb_stage2(
     const BoxDev *__restrict__ boxes, WList wl, BoxState st, Pools p, int fms_ref) {
   constexpr int NT = TX * TY;
   __shared__ double lds[tile2_lds<NT>()];
@@ -528,7 +528,7 @@ template <bool PRED, int ORDER, int RS>
 void b_stages(bnz_batch *c) {
   if (c->nblk[PRED ? KP2 : KC2]) {
     if (c->tile_small) b_stage2<PRED, ORDER, RS, TILE2_SMALL[0], TILE2_SMALL[1]>(c);
-    else b_stage2<PRED, ORDER, RS, TILE2_BIG[0], TILE2_BIG[1]>(c);
+    else b_stage2<PRED, ORDER, RS, TILE2_BIG64[0], TILE2_BIG64[1]>(c);
   }
   b_stage1<PRED, ORDER, RS>(c);
 }
@@ -890,7 +890,7 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   c->tile_small = cells2 <= TILE2_SMALL_CELLS;
   for (BoxDev &d : c->hbox)
     for (int o = 0; o < 2; ++o) {
-      const int *e = c->tile_small ? TILE2_SMALL : TILE2_BIG;
+      const int *e = c->tile_small ? TILE2_SMALL : c->f32 ? TILE2_BIG32 : TILE2_BIG64;
       const Tiling t = tiling2(d.g.nt, d.L[o], o == 0, e[0] - 2, e[1] - 2);
       d.items[o == 0 ? KP2 : KC2] = d.g.dims == 2 ? mkbox(t.o[0], t.n[0], t.o[1], t.n[1], 0, 1)
                                                   : mkbox(0, 0, 0, 0, 0, 0);

@@ -386,7 +386,7 @@ template <bool PRED, int ORDER, int RS>
 void stages(bnz_batch *c) {
   if (c->nblk[PRED ? KP2 : KC2]) {
     if (c->tile_small) stage2<PRED, ORDER, RS, TILE2_SMALL[0], TILE2_SMALL[1]>(c);
-    else stage2<PRED, ORDER, RS, TILE2_BIG[0], TILE2_BIG[1]>(c);
+    else stage2<PRED, ORDER, RS, TILE2_BIG32[0], TILE2_BIG32[1]>(c);
   }
   stage1<PRED, ORDER, RS>(c);
 }

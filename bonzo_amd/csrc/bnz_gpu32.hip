@@ -502,10 +502,10 @@ void stage_fused32(bnz_ctx *c, const Lims &L) {
     else stage3_launch32<PRED, ORDER, BNZ_RS_HLL>(c, L);
   } else if (hlld) {
     if (small) stage2_launch32<PRED, ORDER, BNZ_RS_HLLD, TILE2_SMALL[0], TILE2_SMALL[1]>(c, L);
-    else stage2_launch32<PRED, ORDER, BNZ_RS_HLLD, TILE2_BIG[0], TILE2_BIG[1]>(c, L);
+    else stage2_launch32<PRED, ORDER, BNZ_RS_HLLD, TILE2_BIG32[0], TILE2_BIG32[1]>(c, L);
   } else {
     if (small) stage2_launch32<PRED, ORDER, BNZ_RS_HLL, TILE2_SMALL[0], TILE2_SMALL[1]>(c, L);
-    else stage2_launch32<PRED, ORDER, BNZ_RS_HLL, TILE2_BIG[0], TILE2_BIG[1]>(c, L);
+    else stage2_launch32<PRED, ORDER, BNZ_RS_HLL, TILE2_BIG32[0], TILE2_BIG32[1]>(c, L);
   }
 }
 

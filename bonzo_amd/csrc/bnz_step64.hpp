@@ -214,7 +214,7 @@ __global__ __launch_bounds__(BLK) void k_update(Geo g, const double *w0, const d
 // tile, writes the ghosts and advances the time, so that a step is two
 // launches.
 template <bool PRED, int ORDER, int RS, int TX, int TY>
-__global__ __launch_bounds__(TX *TY, TX *TY >= 512 ? 4 : 2) void k_stage2(Geo g, const double *__restrict__ wf,
+__global__ __launch_bounds__(TX *TY, 2) void k_stage2(Geo g, const double *__restrict__ wf,
                                                    const double *__restrict__ bf,
                                                    const double *w0, const double *b0, double *w1,
                                                    double *b1, Lims L, Tiling tl, Box act,
@@ -355,7 +355,7 @@ void stage_fused(bnz_ctx *c, const Lims &L) {
   do {                                                          \
     if (c->dims == 3) stage3_launch<PRED, ORDER, RS>(c, L);     \
     else if (small) stage2_launch<PRED, ORDER, RS, TILE2_SMALL[0], TILE2_SMALL[1]>(c, L);     \
-    else stage2_launch<PRED, ORDER, RS, TILE2_BIG[0], TILE2_BIG[1]>(c, L);          \
+    else stage2_launch<PRED, ORDER, RS, TILE2_BIG64[0], TILE2_BIG64[1]>(c, L);      \
   } while (0)
   if (rs == BNZ_RS_HLLD) FUSED(BNZ_RS_HLLD);
   else if (rs == BNZ_RS_HLLT) FUSED(BNZ_RS_HLLT);

@@ -99,6 +99,21 @@ __device__ __forceinline__ T from_right(T v, T end = T(0)) {  // row_shl:1
   static_assert(TX == 16, "a row of the tile is a DPP row");
   return dpp_mov<0x101>(end, v);
 }
+// The same in rows of TX lanes, TX any divisor of 64 from 16 up (wave_shr:1,
+// wave_shl:1 and the rows' ends put in by hand); first, last: whether the lane
+// is its row's.
+template <int TX, typename T>
+__device__ __forceinline__ T row_left(T v, T end, bool first) {
+  if (TX == 16) return dpp_mov<0x111>(end, v);
+  const T x = dpp_mov<0x138>(end, v);
+  return first ? end : x;
+}
+template <int TX, typename T>
+__device__ __forceinline__ T row_right(T v, T end, bool last) {
+  if (TX == 16) return dpp_mov<0x101>(end, v);
+  const T x = dpp_mov<0x130>(end, v);
+  return last ? end : x;
+}
 
 // Value of array a (a uniform address) at byte offset o: with a 32-bit offset
 // the load takes its base from scalar registers and one vector register
@@ -371,19 +386,24 @@ inline bool fused_stages(const bnz_ctx *c) {
 }
 
 // Cells up to which a 2D stage takes its small tile (16 x 8: more workgroups
-// on an idle chip; 128^2 20.2 us a step against 23.9 with 16 x 16 tiles),
-// beyond which the big one (32 x 16: fewer rim cells; 32 x 32 is slower, 219
-// against 204 us at 1024^2).
+// on an idle chip; 128^2 18.7 us a step).
 constexpr long TILE2_SMALL_CELLS = 1L << 16;
 
-// Own cells of the tiles, and the partials their launches can leave.
+// Own cells of the tiles, and the partials their launches can leave.  Beyond
+// the small tile FP64 takes 16 x 16 threads, whose 256 registers hold the
+// stencils loaded up front (1024^2 FMA 178 us a step; 32 x 16 threads with the
+// 128 registers that two workgroups a CU leave them 406, one a CU 232, 16 x 16
+// with 168 registers 224), FP32C 32 x 16, which fit there (24 blasts 138 us a
+// step with either; fewer rim cells, 32 x 32 is slower).
 constexpr int TILE3[2] = {16, 16};
-constexpr int TILE2_BIG[2] = {32, 16}, TILE2_SMALL[2] = {16, 8};
+constexpr int TILE2_BIG64[2] = {16, 16}, TILE2_BIG32[2] = {32, 16}, TILE2_SMALL[2] = {16, 8};
 inline long tile_parts(const bnz_ctx *c) {
   const Lims L = integr_lims(c, 0);
   if (c->dims == 3) return tiling3(c, L, true, false, TILE3[0] - 2, TILE3[1] - 2).blocks();
-  return std::max(tiling2(c->nt, L, true, TILE2_BIG[0] - 2, TILE2_BIG[1] - 2).blocks(),
-                  tiling2(c->nt, L, true, TILE2_SMALL[0] - 2, TILE2_SMALL[1] - 2).blocks());
+  long n = 0;
+  for (const int *e : {TILE2_BIG64, TILE2_BIG32, TILE2_SMALL})
+    n = std::max<long>(n, tiling2(c->nt, L, true, e[0] - 2, e[1] - 2).blocks());
+  return n;
 }
 
 // A pending dt over more partials than this is reduced by a launch of its

@@ -47,6 +47,13 @@ __device__ __forceinline__ void copy_ghosts32(const Bnd &b, const Geo &g, const 
       [&](int q, long dst) { a.b1[q * sv + dst] = 0.; });
 }
 
+// The Riemann solver RS on one FP32 face.
+template <int RS>
+__device__ __forceinline__ int solve_face32(float *f, const float *wl, const float *wr, float gam,
+                                            float gm1i, int &ng) {
+  return RS == BNZ_RS_HLLD ? flux_hlld(f, wl, wr, gam, gm1i, &ng) : flux_hll(f, wl, wr, gam, gm1i);
+}
+
 template <int NT>
 struct Tile2Flux32 {
   const float *sx, *sy;
@@ -88,7 +95,7 @@ template <bool PRED, int ORDER, int RS, int TX, int TY, typename BF, class DT>
 __device__ __forceinline__ double stage2_tile32(const Geo &g, const float *__restrict__ wf,
                                                 const BF *__restrict__ bf, const Pred32 &ap,
                                                 const Corr32 &ac, const Lims &L, const DT &step_dt,
-                                                const Box &act, const Bnd &bnd, const Walls &wl,
+                                                const Box &act, const Bnd &bnd, const Walls &walls,
                                                 int fms_ref, int i0, int j0, float *lds, int &ng) {
   constexpr int NT = TX * TY;
   const int t = threadIdx.x, tx = t % TX, ty = t / TX;
@@ -101,16 +108,73 @@ __device__ __forceinline__ double stage2_tile32(const Geo &g, const float *__res
                      j <= L.hi[1] + 1;
   bool gx = false, gy = false;
   int guarded = 0;
-  if (reach && i >= L.lo[0])
-    flux32_face_to<0, ORDER, RS>(g, wf, bf, i, j, 0, guarded, [&](const float *f, long) {
+  // Threads off the grid stand on cell (0, 0), neighbours past the grid's end
+  // are the cell itself: what they give is not used.
+  const int ic = in ? i : 0, jc = in ? j : 0;
+  const long c = (long)jc * g.nt[0] + ic;
+  const bool first = tx == 0, last = tx == TX - 1;
+  const int oxe = first && ic > 0 ? -1 : last && ic < g.nt[0] - 1 ? 1 : 0;
+  const int oyl = jc > 0 ? -g.sy : 0, oyl2 = jc > 1 ? -2 * g.sy : oyl;
+  const int oyr = jc < g.nt[1] - 1 ? g.sy : 0;
+  float wc[NMODE], wl[NMODE], wr[NMODE], f[NMODE];
+  float ym2[NMODE], ym[NMODE], yp[NMODE], xe[NMODE];
+#pragma unroll
+  for (int n = 0; n < NMODE; ++n) {
+    const float *p = wf + n * sv + c;
+    wc[n] = p[0];
+    if (ORDER == 1 && n != BX) xe[n] = p[oxe];
+  }
+  const BF bnx = bf[c], bny = bf[sv + c];
+#pragma unroll
+  for (int n = 0; n < NMODE; ++n)
+    if (n != BY) {
+      const float *p = wf + n * sv + c;
+      ym[n] = p[oyl];
+      if (ORDER == 1) {
+        ym2[n] = p[oyl2];
+        yp[n] = p[oyr];
+      }
+    }
+  // x face: a cell's half slope is formed once and passed to the next lane
+#pragma unroll
+  for (int n = 0; n < NMODE; ++n) {
+    if (n == BX) continue;
+    if (ORDER == 0) {
+      wl[n] = row_left<TX>(wc[n], 0.f, first);
+      wr[n] = wc[n];
+    } else {
+      const float d = vl_half(wc[n] - row_left<TX>(wc[n], xe[n], first),
+                            row_right<TX>(wc[n], xe[n], last) - wc[n]);
+      wl[n] = row_left<TX>(wc[n] + d, 0.f, first);
+      wr[n] = wc[n] - d;
+    }
+  }
+  wl[BX] = wr[BX] = (float)bnx;
+  if (reach && tx > 0 && i >= L.lo[0])
+    if (solve_face32<RS>(f, wl, wr, (float)g.gam, (float)g.gamm1i, guarded)) {
 #pragma unroll
       for (int n = 0; n < 6; ++n) sx[n * NT + t] = f[n];
       sx[6 * NT + t] = f[BY];
       sx[7 * NT + t] = f[BZ];
       gx = true;
-    });
-  if (reach && j >= L.lo[1])
-    flux32_face_to<1, ORDER, RS>(g, wf, bf, i, j, 0, guarded, [&](const float *f, long) {
+    }
+  // y face: both cells' half slopes here
+#pragma unroll
+  for (int n = 0; n < NMODE; ++n) {  // local slot n is variable perm<1>(n)
+    if (n == BX) continue;
+    const int v = perm<1>(n);
+    if (ORDER == 0) {
+      wl[n] = ym[v];
+      wr[n] = wc[v];
+    } else {
+      const float dm = wc[v] - ym[v];
+      wl[n] = ym[v] + vl_half(ym[v] - ym2[v], dm);
+      wr[n] = wc[v] - vl_half(dm, yp[v] - wc[v]);
+    }
+  }
+  wl[BX] = wr[BX] = (float)bny;
+  if (reach && ty > 0 && j >= L.lo[1])
+    if (solve_face32<RS>(f, wl, wr, (float)g.gam, (float)g.gamm1i, guarded)) {
 #pragma unroll
       for (int n = 0; n < NMODE; ++n) {
         if (n == BX) continue;
@@ -118,25 +182,25 @@ __device__ __forceinline__ double stage2_tile32(const Geo &g, const float *__res
         sy[(v < 6 ? v : v == BX ? 6 : 7) * NT + t] = f[n];
       }
       gy = true;
-    });
+    }
   if (own) ng += guarded;
   if (!gx)
     for (int n = 0; n < 8; ++n) sx[n * NT + t] = 0.f;
   if (!gy)
     for (int n = 0; n < 8; ++n) sy[n * NT + t] = 0.f;
-  sc[t] = in ? ec32(wf, sv, (long)j * g.nt[0] + i, 2) : 0.f;
+  sc[t] = -(wc[VX] * wc[BY] - wc[VY] * wc[BX]);  // ec32
   const double dt = step_dt();  // the fluxes did not need it
   __syncthreads();
   if (tx > 0 && ty > 0) {
     const float ez = 0.5f * (-sx[6 * NT + t - TX] - sx[6 * NT + t] + sy[6 * NT + t - 1] +
                              sy[6 * NT + t]) -
                      0.25f * (sc[t - 1] + sc[t] + sc[t - TX - 1] + sc[t - TX]);
-    const bool wx = i == wl.at[0] || i == wl.at[1], wy = j == wl.at[2] || j == wl.at[3];
+    const bool wx = i == walls.at[0] || i == walls.at[1], wy = j == walls.at[2] || j == walls.at[3];
     se[t] = (wx || wy) ? 0.f : ez;
   }
   __syncthreads();
   const Tile2Flux32<NT> fl{sx, sy, t, TX};
-  const Tile2Emf32<NT> em{sx, sy, se, t, TX, (long)g.sy, i, j, wl};
+  const Tile2Emf32<NT> em{sx, sy, se, t, TX, (long)g.sy, i, j, walls};
   if (PRED) {
     if (own) update32_pred_e<2, GeoArr>(g, ap, L, &dt, fl, em, i, j, 0);
     return 0.;
@@ -161,13 +225,6 @@ enum {
   NSLOT3_32 = 30
 };
 enum { UC = 0, UBX = 6, UBY, UBYU, NSLOT3_U = 9 };
-
-// The Riemann solver RS on one FP32 face.
-template <int RS>
-__device__ __forceinline__ int solve_face32(float *f, const float *wl, const float *wr, float gam,
-                                            float gm1i, int &ng) {
-  return RS == BNZ_RS_HLLD ? flux_hlld(f, wl, wr, gam, gm1i, &ng) : flux_hll(f, wl, wr, gam, gm1i);
-}
 
 // One FP32C stage of a column of a 3D grid, as the FP64 stage3_column; the
 // updates are those of update32_pred_e (R = float: hi words and faces of the
