@@ -349,7 +349,7 @@ void stage3_launch(bnz_ctx *c, const Lims &L) {
 
 template <bool PRED, int ORDER>
 void stage_fused(bnz_ctx *c, const Lims &L) {
-  const bool small = c->ncell <= TILE2_SMALL_CELLS;
+  const bool small = tile_small64(c, L, PRED);
   const int rs = rs_kern(c);
 #define FUSED(RS)                                              \
   do {                                                          \

@@ -397,6 +397,19 @@ constexpr long TILE2_SMALL_CELLS = 1L << 16;
 // step with either; fewer rim cells, 32 x 32 is slower).
 constexpr int TILE3[2] = {16, 16};
 constexpr int TILE2_BIG64[2] = {16, 16}, TILE2_BIG32[2] = {32, 16}, TILE2_SMALL[2] = {16, 8};
+
+// Whether an FP64 2D grid takes the small tile: its workgroups find a CU each,
+// or neither tile's do and the grid is below TILE2_SMALL_CELLS.  us per step,
+// FP64, small / big tile (256 CUs): 128^2 (230 / 100 workgroups) 19.1 / 20.6,
+// 160^2 (336 / 144) 25.7 / 20.8, 200^2 (525 / 225) 26.8 / 22.0, 300x190 (726 /
+// 308) 28.4 / 29.4, 250^2 (836 / 361) 29.6 / 29.2.  FP32C, which holds more
+// waves a CU, goes by cells alone: 200^2 21.6 / 23.9, 250^2 23.4 / 23.3.
+inline bool tile_small64(const bnz_ctx *c, const Lims &L, bool pred) {
+  const auto fits = [&](const int *e) {
+    return tiling2(c->nt, L, pred, e[0] - 2, e[1] - 2).blocks() <= c->ncu;
+  };
+  return fits(TILE2_SMALL) || (!fits(TILE2_BIG64) && c->ncell <= TILE2_SMALL_CELLS);
+}
 inline long tile_parts(const bnz_ctx *c) {
   const Lims L = integr_lims(c, 0);
   if (c->dims == 3) return tiling3(c, L, true, false, TILE3[0] - 2, TILE3[1] - 2).blocks();

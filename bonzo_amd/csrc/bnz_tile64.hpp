@@ -213,9 +213,9 @@ __device__ __forceinline__ double stage2_tile(const Geo &g, const double *__rest
       const double f[3] = {bx, by, bz};
       copy_ghosts64(bnd, g, i, j, 0, wn, f, w1, b1);
     };
-    cds = update_cell_e<2, false, true, decltype(em), GeoArr, decltype(fl), false,
+    cds = update_cell_e<2, false, true, decltype(em), GeoArr, decltype(fl),
                         decltype(ghosts)>(g, GeoArr{g}, w0, fl, em, b0, b1, w1, L, &dt, act,
-                                          fms_ref, i, j, 0, 0, ghosts);
+                                          fms_ref, i, j, 0, ghosts);
   }
   return cds;
 }
