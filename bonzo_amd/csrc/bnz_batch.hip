@@ -166,10 +166,12 @@ __global__ __launch_bounds__(BLK) void kb_stage1(const BoxDev *__restrict__ boxe
 // ticket) knows that every other has read the box's dt and folded its CFL
 // maximum, and does for the box what time_dt_block does.
 // 256 tubes of 64 to 1024 cells to t = 0.1: 27.1 -> 25.6 ms against a step and
-// a ghost launch; with device-wide fences around the ticket instead 36.0 (each
-// writes back an L2).
+// a ghost launch, 22.7 without the graph (advance_steps); with device-wide
+// fences around the ticket instead 36.0 (each writes back an L2).  Three waves
+// a SIMD (170 registers): 512 tubes of 64 to 4096 cells 42.5 us a step; with
+// two 46.6, with four, which spill, 65.6.
 template <int ORDER, int RS>
-__global__ __launch_bounds__(BLK) void kb_step1(const BoxDev *__restrict__ boxes, WList wl,
+__global__ __launch_bounds__(BLK, 3) void kb_step1(const BoxDev *__restrict__ boxes, WList wl,
                                                 BoxState st, Pools p, int fms_ref, double cour) {
   __shared__ double lds[TUBE_SLOTS * BLK];
   __shared__ double red[BLK / 64];
@@ -678,8 +680,11 @@ void drop_graph(bnz_batch *c) {
 // Steps until every box has reached its t_max, or max_steps; n: the steps
 // launched.
 int advance_steps(bnz_batch *c, int max_steps, int use_graph, int &n) {
-  if (use_graph && c->exec && c->graph_b != c->P.b) drop_graph(c);
-  if (use_graph && !c->exec) {
+  // a step that is one launch goes out directly, in the same pairs: a replay of
+  // a graph of two costs 3 us a step more
+  const bool replay = use_graph && !(c->step1 && !c->f32);
+  if (replay && c->exec && c->graph_b != c->P.b) drop_graph(c);
+  if (replay && !c->exec) {
     c->graph_b = c->P.b;
     BCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     b_step(c);
@@ -702,7 +707,12 @@ int advance_steps(bnz_batch *c, int max_steps, int use_graph, int &n) {
   auto chunk = [&](int slot) -> int {
     if (use_graph) {
       for (int r = 0; r < REPLAYS && (max_steps <= 0 || n < max_steps); ++r) {
-        BCHK(c, hipGraphLaunch(c->exec, c->stream));
+        if (replay) {
+          BCHK(c, hipGraphLaunch(c->exec, c->stream));
+        } else {
+          b_step(c);
+          b_step(c);
+        }
         n += 2;
       }
     } else {

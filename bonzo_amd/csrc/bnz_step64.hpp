@@ -76,15 +76,18 @@ __global__ __launch_bounds__(BLK) void k_flux3(Geo g, const double *__restrict__
 // by then every workgroup has read; the partials go to another buffer than
 // dtf's.  As three launches (dt, step, ghosts) a step of 512 cells took 12.7 us
 // and takes 10.4 (FMA 11.8, 9.7), some 5 of them from launch to launch; with
-// every phase of step1_block loading what it needs 11.4.
+// every phase of step1_block loading what it needs 11.4.  Three waves a SIMD: a
+// million cells, where the partials have a launch of their own, 71.8 us a step
+// for 74.6 (FMA 62.4, 66.4); reduced by every workgroup 82.8.
 template <int ORDER, int RS, bool CP = false, bool FOLD = false>
-__global__ __launch_bounds__(BLK) void k_step1(Geo g, const double *__restrict__ w,
+__global__ __launch_bounds__(BLK, 3) void k_step1(Geo g, const double *__restrict__ w,
                                                const double *__restrict__ bf,
                                                double *__restrict__ wout,
                                                double *__restrict__ bout,
                                                const double *__restrict__ fx_old,
                                                double *dev, int fms_ref,
-                                               DtFold dtf, Bnd bnd, int *ticket,
+                                               DtFold dtf, const double *carry, int ncarry,
+                                               Bnd bnd, int *ticket,
                                                double *__restrict__ part) {
   __shared__ double lds[TUBE_SLOTS * BLK];
   const int i0 = blockIdx.x * STEP1_CELLS;
@@ -103,10 +106,10 @@ __global__ __launch_bounds__(BLK) void k_step1(Geo g, const double *__restrict__
       for (int a = 0; a < 3; ++a) bout[a * g.sv + i] = bf[a * g.sv + i];
     }
     if (!FOLD) return;
-    // and the partials
+    // and its partials
     cds = 0.;
-    for (int q = blockIdx.x * BLK + threadIdx.x; q < dtf.npart; q += gridDim.x * BLK)
-      cds = fmax(cds, dtf.part[q]);
+    for (int q = blockIdx.x * BLK + threadIdx.x; q < ncarry; q += gridDim.x * BLK)
+      cds = fmax(cds, carry[q]);
   }
   block_max_to(cds, part);
   if (FOLD && threadIdx.x == 0 && dt != 0.) {
@@ -481,16 +484,20 @@ void launch_update(bnz_ctx *c, bool pred, const Lims &L, const double *we = null
 }
 
 // A 1D step as one fused launch (k_step1): w, b -> ws, bs, then swapped.
+constexpr int STEP1_FOLD_PARTS = BLK;
 template <int ORDER, int RS>
 void step1_launch(bnz_ctx *c) {
   const int nb = (c->nt[0] + STEP1_CELLS - 1) / STEP1_CELLS;
   const bool fold = step1_folds(c);
+  // many partials are reduced by a launch of their own, not by every workgroup
+  const DtFold state = fold ? c->pdt : DtFold{};
+  if (fold && state.npart > STEP1_FOLD_PARTS) flush_dt(c);
   const DtFold dtf = fold ? take_dt(c) : DtFold{};
   Launch t(c, "step1");
 #define STEP1(CP, FOLD)                                                                         \
   hipLaunchKernelGGL((k_step1<ORDER, RS, CP, FOLD>), dim3(nb), dim3(BLK), 0, c->stream, c->g,   \
-                     c->w, c->b, c->ws, c->bs, c->fx, c->dev, cfl_mode(c), dtf,                 \
-                     bnd_of(c), c->ticket, fold ? c->part2 : c->part)
+                     c->w, c->b, c->ws, c->bs, c->fx, c->dev, cfl_mode(c), dtf, state.part,     \
+                     state.npart, bnd_of(c), c->ticket, fold ? c->part2 : c->part)
   if (ORDER == 1 && c->p.char_proj) {
     if (fold) STEP1(true, true);
     else STEP1(true, false);

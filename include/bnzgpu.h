@@ -315,7 +315,8 @@ int bnz_batch_download(bnz_batch *b, int box, double *prim, double *bfld);
 int bnz_batch_init_state(bnz_batch *b);
 /* Steps until every box has reached its t_max, or max_steps (> 0) step
    launches.  use_graph: replay a hipGraph holding two captured steps (steps
-   are then launched in pairs).  Steps go out in chunks (four pairs, or one
+   are then launched in pairs; those of an FP64 batch of 1D boxes, one launch
+   each, go out directly in the same pairs).  Steps go out in chunks (four pairs, or one
    eager step) and the host reads a chunk's count of running boxes while
    the next chunk runs, so up to one chunk may run after the last box
    finished (a box at its t_max idles).  An FP64 batch of 1D boxes of at most
