@@ -397,8 +397,8 @@ struct Corr32 {
 // predictor.
 // SPLIT (the corrector of a fused 1D step): the new hi and lo words go to
 // uh1 and ul1 instead of back to a.uh and a.ul.  copy gets the new hi words,
-// prim and lower faces of an updated cell (the ghost images).  lo_only: a
-// ghost cell whose other words come from the fill in the same launch.
+// prim and lower faces of an updated cell (the ghost images).  Ghost cells keep
+// their low words (see Ghost32).
 struct NoCopy32 {
   __device__ __forceinline__ void operator()(const float *, const double *, const double *) const {}
 };
@@ -408,8 +408,7 @@ __device__ __forceinline__ double update32_corr_e(const Geo &g, const Corr32 &a,
                                                   int fms_ref, const FL &fl, const EM &em, int i,
                                                   int j, int k, float *uh1 = nullptr,
                                                   float *ul1 = nullptr,
-                                                  const COPY &copy = COPY{},
-                                                  bool lo_only = false) {
+                                                  const COPY &copy = COPY{}) {
   const long c = ((long)k * g.nt[1] + j) * g.nt[0] + i, sv = g.sv;
   double cdsmax = 0.;
   const double dt = dts[0];
@@ -457,28 +456,21 @@ __device__ __forceinline__ double update32_corr_e(const Geo &g, const Corr32 &a,
   else
     u[BZ] = lo[2];
   cons2prim(wv, u, g.gam);
-  if (lo_only) {
-    if (ro.cell) {
-#pragma unroll
-      for (int n = 0; n < NMODE - 3; ++n) a.ul[n * sv + c] = nl[n];
-    }
-    return 0.;
-  }
   if (ro.fX) a.b1[c] = lo[0];
   if (ro.fY) a.b1[sv + c] = lo[1];
   if (ro.fZ) a.b1[2 * sv + c] = lo[2];
   if (ro.cell) {
+    const bool active = i >= act.lo[0] && i < act.lo[0] + act.n[0] && j >= act.lo[1] &&
+                        j < act.lo[1] + act.n[1] && k >= act.lo[2] && k < act.lo[2] + act.n[2];
 #pragma unroll
     for (int n = 0; n < NMODE - 3; ++n) {
       (SPLIT ? uh1 : a.uh)[n * sv + c] = nh[n];
-      (SPLIT ? ul1 : a.ul)[n * sv + c] = nl[n];
+      if (active) (SPLIT ? ul1 : a.ul)[n * sv + c] = nl[n];
     }
 #pragma unroll
     for (int n = 0; n < NMODE; ++n) a.w32[n * sv + c] = (float)wv[n];
     copy(nh, wv, lo);
-    if (i >= act.lo[0] && i < act.lo[0] + act.n[0] && j >= act.lo[1] &&
-        j < act.lo[1] + act.n[1] && k >= act.lo[2] && k < act.lo[2] + act.n[2])
-      cdsmax = cds_cell_g(gm, g, wv, fms_ref, i, j, k);
+    if (active) cdsmax = cds_cell_g(gm, g, wv, fms_ref, i, j, k);
   }
   return cdsmax;
 }
@@ -579,9 +571,11 @@ __device__ __forceinline__ double cfl32_cell(const Geo &g, const float *__restri
 
 // The ghost fill of the FP32C state: conserved hi words (uh) and FP32 prim
 // (w32) of every variable, and the face fields.  The low words (ul) get no
-// ghosts: only the corrector reads them, and of the cells it updates only the
-// active ones keep their result (the fill overwrites the others' hi words and
-// prim after the step).
+// ghosts and no ghost cell's are ever stored after init or load: only the
+// corrector reads low words, and of the cells it updates only the active ones
+// keep their result (the fill overwrites the others' hi words and prim).  A
+// fused 2D stage writes the ghosts' hi words from other workgroups, so nothing
+// formed from them there could be kept.
 constexpr int NGHOST32 = 6 + NMODE;
 struct Ghost32 {
   float *a[NGHOST32];  // uh (6), w32 (9)

@@ -88,9 +88,11 @@ constexpr int tile2_lds32() {
 }
 
 // One FP32C stage over one 2D tile (stage2_tile).  The fluxes come from the
-// stage's FP32 prim wf and faces bf; ap / ac as in the separate updates, ac.b1
-// and the words the corrector writes are read by no other tile's call.  ng
-// counts the guarded faces of the cells the tile owns.
+// stage's FP32 prim wf and faces bf; ap / ac as in the separate updates.  As
+// there the corrector updates the active cells only and writes their ghosts:
+// it reads the words of its own active cells, which no other tile writes, and
+// wf, bf and ac.b, which no corrector writes.  ng counts the guarded faces of
+// the cells the tile owns.
 template <bool PRED, int ORDER, int RS, int TX, int TY, typename BF, class DT>
 __device__ __forceinline__ double stage2_tile32(const Geo &g, const float *__restrict__ wf,
                                                 const BF *__restrict__ bf, const Pred32 &ap,
@@ -206,14 +208,13 @@ __device__ __forceinline__ double stage2_tile32(const Geo &g, const float *__res
     return 0.;
   }
   double cds = 0.;
-  if (own) {
-    const bool active = i >= act.lo[0] && i < act.lo[0] + act.n[0] && j >= act.lo[1] &&
-                        j < act.lo[1] + act.n[1];
+  if (own && i >= act.lo[0] && i < act.lo[0] + act.n[0] && j >= act.lo[1] &&
+      j < act.lo[1] + act.n[1]) {
     const auto ghosts = [&](const float *uh, const double *w, const double *f) {
       if (near_side(bnd, i, j, 0)) copy_ghosts32(bnd, g, ac, i, j, 0, uh, w, f);
     };
     cds = update32_corr_e<2, GeoArr, decltype(fl), decltype(em), false, decltype(ghosts)>(
-        g, ac, L, &dt, act, fms_ref, fl, em, i, j, 0, nullptr, nullptr, ghosts, !active);
+        g, ac, L, &dt, act, fms_ref, fl, em, i, j, 0, nullptr, nullptr, ghosts);
   }
   return cds;
 }
@@ -512,8 +513,10 @@ __device__ __forceinline__ double stage3_column32(const Geo &g, const float *__r
           for (int n = 0; n < 6; ++n) {
             float h, l;
             split(uv[n], h, l);
-            if (active) put(ac.uh + n * sv, 4u * om, h);
-            put(ac.ul + n * sv, 4u * om, l);
+            if (active) {
+              put(ac.uh + n * sv, 4u * om, h);
+              put(ac.ul + n * sv, 4u * om, l);
+            }
           }
         }
         float *wo = PRED ? ap.ws : ac.w32;
