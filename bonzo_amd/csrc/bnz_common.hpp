@@ -656,6 +656,17 @@ inline void build_ghosts(const int nt[3], int dims, int ng, const int bc[6], lon
             mf[a][idx] = 2 * a1 - idx;
             ff[a][idx] = 1;
           }
+          if (mf[a][0] > a2 && bc[2 * a + 1] >= 0) {
+            // just ng cells: the mirror face is one the high side fills, so it
+            // is taken as that side leaves it (0: a wall)
+            if (bc[2 * a + 1] == BNZ_BC_OUTFLOW) {
+              mf[a][0] = a2;
+            } else {
+              mf[a][0] = 0;
+              ff[a][0] = 0;
+              zf[a][0] = 1;
+            }
+          }
         } else {
           for (int idx = a2 + 2; idx < N; ++idx) {
             mf[a][idx] = 2 * a2 + 2 - idx;

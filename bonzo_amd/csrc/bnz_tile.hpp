@@ -175,11 +175,19 @@ struct Bnd {
   int plain;         // no reflecting side
 };
 
+// Whether the low ghosts of an axis mirror a face past its active cells: with a
+// reflecting low side and just ng cells, ghost face a1 - ng mirrors face
+// a2 + 1, which the high side sets.  It then mirrors what that side copies
+// there: face a2 with outflow, else a wall face, 0 (build_ghosts does the same).
+__host__ __device__ __forceinline__ bool low_mirrors_end(const Bnd &b, int axis) {
+  return b.flag[2 * axis] == BNZ_BC_REFLECT && b.a2[axis] - b.a1[axis] + 1 == b.ng;
+}
+
 // Images of index x along one axis, bit 0 x itself, bit 1 + g the low ghost
 // a1 - ng + g, bit 1 + ng + g the high ghost a2 + 1 + g.  FACE: the images of
 // a face index of the axis's own normal field (mirrored about the wall face).
 template <bool FACE>
-__device__ __forceinline__ unsigned images(const Bnd &b, int axis, int x) {
+__host__ __device__ __forceinline__ unsigned images(const Bnd &b, int axis, int x) {
   unsigned m = 1u;
   if (axis >= b.dims) return m;
   const int a1 = b.a1[axis], a2 = b.a2[axis], ng = b.ng, n = a2 - a1 + 1;
@@ -192,6 +200,7 @@ __device__ __forceinline__ unsigned images(const Bnd &b, int axis, int x) {
   }
   if (hi == BNZ_BC_OUTFLOW) {
     if (x == a2) m |= ((1u << ng) - 1) << (1 + ng);
+    if (FACE && x == a2 && low_mirrors_end(b, axis)) m |= 2u;
   } else {
     const int q = hi == BNZ_BC_PERIODIC ? x + n : FACE ? 2 * a2 + 2 - x : 2 * a2 + 1 - x;
     const int q0 = (FACE && hi == BNZ_BC_REFLECT) ? a2 + 2 : a2 + 1;
@@ -201,7 +210,8 @@ __device__ __forceinline__ unsigned images(const Bnd &b, int axis, int x) {
 }
 
 // Index of image bit s of x, and whether that side mirrors it.
-__device__ __forceinline__ int image_at(const Bnd &b, int axis, int s, int x, bool &flip) {
+__host__ __device__ __forceinline__ int image_at(const Bnd &b, int axis, int s, int x,
+                                                 bool &flip) {
   flip = false;
   if (s == 0) return x;
   const int g = s - 1;
@@ -212,8 +222,9 @@ __device__ __forceinline__ int image_at(const Bnd &b, int axis, int s, int x, bo
 // f(cell index, flips) for every combination of images but the cell itself;
 // bit a of flips: mirrored along axis a.
 template <class F>
-__device__ __forceinline__ void each_image(const Bnd &b, const Geo &g, const unsigned m[3], int i,
-                                           int j, int k, const F &f) {
+__host__ __device__ __forceinline__ void each_image(const Bnd &b, const Geo &g,
+                                                    const unsigned m[3], int i, int j, int k,
+                                                    const F &f) {
   for (unsigned mz = m[2]; mz; mz &= mz - 1) {
     bool fz, fy, fx;
     const int kk = image_at(b, 2, __builtin_ctz(mz), k, fz);
@@ -230,7 +241,7 @@ __device__ __forceinline__ void each_image(const Bnd &b, const Geo &g, const uns
 }
 
 // Whether active cell (i, j, k) has images, or a wall face of its own.
-__device__ __forceinline__ bool near_side(const Bnd &b, int i, int j, int k) {
+__host__ __device__ __forceinline__ bool near_side(const Bnd &b, int i, int j, int k) {
   const int x[3] = {i, j, k};
   bool any = false;
   for (int a = 0; a < 3; ++a)
@@ -245,9 +256,9 @@ __device__ __forceinline__ bool near_side(const Bnd &b, int i, int j, int k) {
 // Together over the active cells this writes every ghost cell as build_ghosts
 // and the ghost fill do; each target has one source.
 template <class CELLS, class FACE, class WALL>
-__device__ __forceinline__ void scatter_ghosts(const Bnd &b, const Geo &g, int i, int j, int k,
-                                               const CELLS &cells, const FACE &face,
-                                               const WALL &wall) {
+__host__ __device__ __forceinline__ void scatter_ghosts(const Bnd &b, const Geo &g, int i, int j,
+                                                        int k, const CELLS &cells,
+                                                        const FACE &face, const WALL &wall) {
   const unsigned m[3] = {images<false>(b, 0, i), images<false>(b, 1, j), images<false>(b, 2, k)};
   each_image(b, g, m, i, j, k, cells);
   const int x[3] = {i, j, k};
@@ -260,10 +271,13 @@ __device__ __forceinline__ void scatter_ghosts(const Bnd &b, const Geo &g, int i
     f[a] = a == 0 ? images<true>(b, 0, i) : a == 1 ? images<true>(b, 1, j) : images<true>(b, 2, k);
     const bool zlo = b.flag[2 * a] == BNZ_BC_REFLECT && x[a] == b.a1[a];
     const bool zhi = b.flag[2 * a + 1] == BNZ_BC_REFLECT && x[a] == b.a2[a];
+    const bool zend = b.flag[2 * a + 1] != BNZ_BC_OUTFLOW && x[a] == b.a2[a] &&
+                      low_mirrors_end(b, a);
     each_image(b, g, f, i, j, k,
                [&](long dst, unsigned flips) { face(a, dst, ((flips >> a) & 1u) != 0); });
-    if (zlo || zhi) {
-      // the wall face itself and its images along the other axes
+    if (zlo || zhi || zend) {
+      // the wall face itself (zend: its mirror image past the low ghosts) and
+      // its images along the other axes
       unsigned o[3] = {m[0], m[1], m[2]};
       o[a] = 1u;
       const long step = a == 0 ? 1 : a == 1 ? g.sy : g.sz;
@@ -275,6 +289,11 @@ __device__ __forceinline__ void scatter_ghosts(const Bnd &b, const Geo &g, int i
       if (zhi) {
         wall(a, self + step);
         each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst + step); });
+      }
+      if (zend) {
+        const long back = (b.a2[a] - b.a1[a] + b.ng) * step;
+        wall(a, self - back);
+        each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst - back); });
       }
     }
   }

@@ -133,3 +133,40 @@ def test_fused_matches_the_oracle(n, rs, kw):
     assert np.array_equal(gp[act], o.prim[act])
     assert np.array_equal(gb[act], o.bfld[act])
     o.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32c"])
+@pytest.mark.parametrize("hi", [1, 2])
+@pytest.mark.parametrize("n,axis", [((3, 1, 1), 0), ((3, 40, 1), 0), ((40, 3, 1), 1)])
+def test_ghosts_of_the_shortest_walled_axis(n, axis, hi, prec):
+    """A reflecting low side on an axis of just ng cells: its outermost ghost
+    face mirrors a face that the high side fills, on every route."""
+    from bonzo_amd._lib import Batch
+    from tests.test_gpu_batch import box_desc
+    print(f"case: {n} axis {axis} hi {hi} {prec}", flush=True)
+    bc = [0] * 6
+    bc[2 * axis], bc[2 * axis + 1] = 2, hi
+    s, prim, bfld = _state(*n, 3, 71)
+    outs = []
+    for tune in ((0, 0, 0), (1, 1, 1)):
+        outs.append(_run(s, prim, bfld, 4, tune=tune, bc=tuple(bc), precision=prec)[:2])
+    if prec == "fp64" and n[1] == 1:
+        out = outs[1]  # one launch a step (k_step1), and in a batch beside a long box
+        s2, prim2, bfld2 = _state(600, 1, 1, 3, 72)
+        b = Batch([box_desc(s, tuple(bc), 1e9), box_desc(s2, (0,) * 6, 1e9)])
+        b.upload(1, prim2, bfld2)
+    else:
+        out = outs[0]
+        b = Batch([box_desc(s, tuple(bc), 1e9)], precision=prec)
+    b.upload(0, prim, bfld)
+    b.init_state()
+    b.advance(max_steps=3, use_graph=False)
+    outs.append(b.download(0))
+    b.close()
+    assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+    for _, face in outs:
+        f = np.moveaxis(face[axis], 2 - axis, 0)  # the axis first
+        other = [slice(3, -3) if m > 1 else slice(None) for m in f.shape[1:]]
+        last = f[5] if hi == 1 else 0.0 * f[5]
+        assert np.array_equal(f[0], -last)
+        assert np.abs(f[5][tuple(other)]).min() > 0.0
