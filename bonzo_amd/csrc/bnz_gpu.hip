@@ -963,6 +963,8 @@ int bnz_upload(bnz_ctx *c, const double *prim, const double *bfld) {
   HIPCHK(c, c->link.up(c->p.device, c->stream, seg, k));
   if (!bfld && c->p.hydro)
     HIPCHK(c, hipMemsetAsync(c->b, 0, 3 * c->ncell * sizeof(double), c->stream));
+  // the call waits for the work queued before it, and reports its errors
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   // the uploaded state has no ghosts, cell-centred field or FP32C words yet
   c->ready = false;
   return BNZ_OK;

@@ -90,3 +90,27 @@ def test_run_between_transfers_matches_one_run():
         assert np.array_equal(x, y)
     a.close()
     c.close()
+
+
+@pytest.mark.parametrize("n", [20, 128, 300])
+def test_upload_waits_for_the_queued_work(n):
+    """Plain, one-launch and chunked uploads alike return when the steps queued
+    before them have ended."""
+    import time
+    from bonzo_amd._lib import Context
+    print(f"case: {n}^2", flush=True)
+    s, prim, bfld = P.orszag_tang(n)
+    g = Context(n, n)
+    g.upload(prim, bfld)
+    g.init_state()
+    g.run_steps(50)
+    g.synchronize()
+    g.run_steps(4000)  # some 80 ms
+    t0 = time.perf_counter()
+    g.upload(prim, bfld)
+    t1 = time.perf_counter()
+    g.synchronize()
+    t2 = time.perf_counter()
+    g.close()
+    # what is left of the queue: an idle stream's wait, not thousands of steps
+    assert t2 - t1 < 0.25 * (t1 - t0) + 1e-3, (t1 - t0, t2 - t1)
