@@ -349,6 +349,7 @@ struct bnz_ctx {
   int i1, i2, j1, j2, k1, k2;
   long ncell = 0;
   int ncu = 256;  // compute units of the device
+  bool columns = false;  // 3D: the stages run as columns (columns_pay)
   hipStream_t stream = nullptr;
   double *w = nullptr, *ws = nullptr, *b = nullptr, *bs = nullptr;
   double *fx = nullptr, *fy = nullptr, *fz = nullptr, *ee = nullptr;

@@ -834,6 +834,7 @@ int bnz_create(const bnz_params *p, bnz_ctx **out) {
   for (int q = 0; q < 2; ++q) HIPCHK(c, hipEventCreateWithFlags(&c->hev[q], hipEventDisableTiming));
   const size_t cells = (size_t)c->ncell;
   c->f32 = (p->precision == BNZ_PREC_FP32C);
+  c->columns = c->dims == 3 && columns_pay(c);
   // FP64 prim and faces always exist (upload, init, download); the FP64
   // work arrays only for the FP64 step
   std::vector<double **> bufs9 = {&c->w}, bufs3 = {&c->b, &c->bs};

@@ -496,7 +496,7 @@ void stage3_launch32(bnz_ctx *c, const Lims &L) {
 
 template <bool PRED, int ORDER>
 void stage_fused32(bnz_ctx *c, const Lims &L) {
-  const bool small = c->ncell <= TILE2_SMALL_CELLS, hlld = c->p.rsolver == BNZ_RS_HLLD;
+  const bool small = tile_small32(c, L, PRED), hlld = c->p.rsolver == BNZ_RS_HLLD;
   if (c->dims == 3) {
     if (hlld) stage3_launch32<PRED, ORDER, BNZ_RS_HLLD>(c, L);
     else stage3_launch32<PRED, ORDER, BNZ_RS_HLL>(c, L);

@@ -353,6 +353,7 @@ constexpr long STAGE3_RUN_CELLS = 1L << 23;
 struct Tiling3 {
   int o[3], n[3], nz, top;  // origin, tiles per axis, planes per run, last plane
   int runs;                 // workgroups in run_block order
+  long cost;                // planes walked one after the other, over the rounds
   int blocks() const { return n[0] * n[1] * n[2]; }
 };
 inline Tiling3 tiling3(const bnz_ctx *c, const Lims &L, bool pred, bool active, int ex,
@@ -376,7 +377,7 @@ inline Tiling3 tiling3(const bnz_ctx *c, const Lims &L, bool pred, bool active, 
         const int run = (planes + q - 1) / q, runs = (planes + run - 1) / run;
         const long cost = (cols * runs + slots - 1) / slots * (run + 2);
         if (!best || cost < best) {
-          best = cost;
+          best = t.cost = cost;
           t.nz = run;
           t.n[2] = runs;
         }
@@ -393,15 +394,51 @@ inline Tiling3 tiling3(const bnz_ctx *c, const Lims &L, bool pred, bool active, 
 constexpr long STAGE3_MAX_CELLS = 1L << 29;
 constexpr long STAGE3_MIN_CELLS64 = 400000, STAGE3_MIN_CELLS32 = 1L << 20;
 
-// Grids whose stages run as fused passes: 2D and 3D Van-Leer steps in the
-// default placement (bnz_set_tuning 0, 0, 0).  The upwind EMF, characteristic
-// limiting and user boundaries keep the separate kernels.
-inline bool fused_stages(const bnz_ctx *c) {
-  if (c->dims == 3 && (c->ncell > STAGE3_MAX_CELLS ||
-                       c->ncell < (c->f32 ? STAGE3_MIN_CELLS32 : STAGE3_MIN_CELLS64)))
+constexpr int TILE3[2] = {16, 16};
+
+// Whether a 3D grid's stages run as columns.  Columns take as long as the planes
+// their rounds walk (Tiling3::cost), the separate kernels as long as the grid
+// has cells: columns pay where the cells are at least the given share of the
+// cells that the walked planes have room for.  Thin sides, which leave most of
+// a tile idle, and grids whose last round is nearly empty fall below it.  us per
+// step, separate / columns, over 101 shapes of 3 to 30000 cells a side: no shape
+// is more than 6 % slower than with the better of the two.  share, FP64: 0.40
+// (3x3x30000) 899 / 1464, 0.59 (30x30x1000) 495 / 521, 0.64 (200x16x200) 352 /
+// 360, 0.66 (200x8x300) 321 / 283, 0.87 (128^3) 917 / 731; FMA: 0.53 0.93 times
+// as fast, 0.59 1.02; FP32C: 0.62 (1000x3x1000) 1863 / 2640, 0.64 (5x320x300) 265
+// / 326, 0.71 (96^3) 237 / 261, 0.73 (322x337x33) 1.06 times as fast, 0.74 (112^3)
+// 409 / 410, 0.83 (104^3) 295 / 283.
+inline bool columns_pay(const bnz_ctx *c) {
+  if (c->ncell > STAGE3_MAX_CELLS ||
+      c->ncell < (c->f32 ? STAGE3_MIN_CELLS32 : STAGE3_MIN_CELLS64))
     return false;
-  return c->dims >= 2 && !c->p.tintegr && !c->p.ct_upwind && !c->p.char_proj && c->npass == 0 &&
-         c->flux_chunk == 0 && c->emf_chunk == 0 && c->update_chunk == 0;
+  const int ex = TILE3[0] - 2, ey = TILE3[1] - 2;
+  const long cost = tiling3(c, integr_lims(c, 0), true, !c->f32, ex, ey).cost +
+                    tiling3(c, integr_lims(c, c->order), false, !c->f32, ex, ey).cost;
+  const double room = (double)ex * ey * STAGE3_PER_CU * c->ncu * (double)cost;
+  const double share = c->f32 ? 0.725 : c->p.precision == BNZ_PREC_FP64_FMA ? 0.55 : 0.63;
+  return 2. * (double)c->ncell >= share * room;
+}
+
+// Whether a 2D grid is too thin for tiles: long grids some ten cells across
+// with their ghosts, where a tile's row or column is mostly idle.  us per step,
+// separate / tiles: FP64 200000x3 516 / 536, 3x200000 593 / 560, 4x150000 472 /
+// 424 (FMA 200000x3 503 / 500); FP32C 3x22222 62 / 68, 4x20000 60 / 63, 5x18181
+// 61 / 58, 22222x3 57 / 38 (its tile is wider than high).  Short grids are bound
+// by their launches, of which tiles have fewer (FP32C 3x2000 27 / 22).
+inline bool thin2(const bnz_ctx *c) {
+  if (c->f32) return c->nt[0] <= 10 && c->ncell > 1L << 17;
+  return c->nt[1] <= 9 && c->ncell > 1L << 20 && c->p.precision == BNZ_PREC_FP64;
+}
+
+// Grids whose stages run as fused passes: 2D and 3D Van-Leer steps in the
+// default placement (bnz_set_tuning 0, 0, 0) of grids that fill their tiles.
+// The upwind EMF, characteristic limiting and user boundaries keep the separate
+// kernels.
+inline bool fused_stages(const bnz_ctx *c) {
+  return c->dims >= 2 && !(c->dims == 3 ? !c->columns : thin2(c)) && !c->p.tintegr &&
+         !c->p.ct_upwind && !c->p.char_proj && c->npass == 0 && c->flux_chunk == 0 &&
+         c->emf_chunk == 0 && c->update_chunk == 0;
 }
 
 // Cells up to which a 2D stage takes its small tile (16 x 8: more workgroups
@@ -414,27 +451,54 @@ constexpr long TILE2_SMALL_CELLS = 1L << 16;
 // 128 registers that two workgroups a CU leave them 406, one a CU 232, 16 x 16
 // with 168 registers 224), FP32C 32 x 16, which fit there (24 blasts 138 us a
 // step with either; fewer rim cells, 32 x 32 is slower).
-constexpr int TILE3[2] = {16, 16};
 constexpr int TILE2_BIG64[2] = {16, 16}, TILE2_BIG32[2] = {32, 16}, TILE2_SMALL[2] = {16, 8};
 
+// Threads of a launch of tiles of e[0] x e[1] threads.
+inline long tile_threads(const int *nt, const Lims &L, bool pred, const int *e) {
+  return (long)tiling2(nt, L, pred, e[0] - 2, e[1] - 2).blocks() * e[0] * e[1];
+}
+
 // Whether an FP64 2D grid takes the small tile: its workgroups find a CU each,
-// or neither tile's do and the grid is below TILE2_SMALL_CELLS.  us per step,
-// FP64, small / big tile (256 CUs): 128^2 (230 / 100 workgroups) 19.1 / 20.6,
-// 160^2 (336 / 144) 25.7 / 20.8, 200^2 (525 / 225) 26.8 / 22.0, 300x190 (726 /
-// 308) 28.4 / 29.4, 250^2 (836 / 361) 29.6 / 29.2.  FP32C, which holds more
-// waves a CU, goes by cells alone: 200^2 21.6 / 23.9, 250^2 23.4 / 23.3.
+// or neither tile's do and the grid is below TILE2_SMALL_CELLS or covered with
+// four fifths of the threads (a thin grid of 12 rows: 18 with ghosts are 3
+// rows of small tiles, 2 of big).  us per step, FP64, small / big tile (256
+// CUs): 128^2 (230 / 100 workgroups) 19.1 / 20.6, 160^2 (336 / 144) 25.7 / 20.8,
+// 200^2 (525 / 225) 26.8 / 22.0, 300x190 (726 / 308) 28.4 / 29.4, 250^2 (836 /
+// 361) 29.6 / 29.2, 11111x12 62.8 / 77.3, 83333x12 343 / 501 (separate kernels
+// 458).
 inline bool tile_small64(const bnz_ctx *c, const Lims &L, bool pred) {
   const auto fits = [&](const int *e) {
     return tiling2(c->nt, L, pred, e[0] - 2, e[1] - 2).blocks() <= c->ncu;
   };
-  return fits(TILE2_SMALL) || (!fits(TILE2_BIG64) && c->ncell <= TILE2_SMALL_CELLS);
+  if (fits(TILE2_SMALL)) return true;
+  if (fits(TILE2_BIG64)) return false;
+  return c->ncell <= TILE2_SMALL_CELLS ||
+         5 * tile_threads(c->nt, L, pred, TILE2_SMALL) <=
+             4 * tile_threads(c->nt, L, pred, TILE2_BIG64);
 }
+
+// Whether an FP32C one does, which holds more waves a CU: by cells (200^2 21.6 /
+// 23.9, 250^2 23.4 / 23.3), or where it takes nine tenths of the threads, as on
+// grids that use little of the big tile's rows of 32 (8x14285 45 / 57, 8x107142
+// 216 / 357, separate 305; 10x93750 231 / 305, 12x83333 294 / 292).
+inline bool tile_small32(const bnz_ctx *c, const Lims &L, bool pred) {
+  return c->ncell <= TILE2_SMALL_CELLS ||
+         10 * tile_threads(c->nt, L, pred, TILE2_SMALL) <=
+             9 * tile_threads(c->nt, L, pred, TILE2_BIG32);
+}
+
+// Partials that the launches of a grid's stages can leave, whatever the tile.
 inline long tile_parts(const bnz_ctx *c) {
-  const Lims L = integr_lims(c, 0);
-  if (c->dims == 3) return tiling3(c, L, true, false, TILE3[0] - 2, TILE3[1] - 2).blocks();
   long n = 0;
-  for (const int *e : {TILE2_BIG64, TILE2_BIG32, TILE2_SMALL})
-    n = std::max<long>(n, tiling2(c->nt, L, true, e[0] - 2, e[1] - 2).blocks());
+  for (const bool pred : {true, false}) {
+    const Lims L = integr_lims(c, pred ? 0 : c->order);
+    if (c->dims == 3) {
+      n = std::max<long>(n, tiling3(c, L, pred, !c->f32, TILE3[0] - 2, TILE3[1] - 2).blocks());
+      continue;
+    }
+    for (const int *e : {TILE2_BIG64, TILE2_BIG32, TILE2_SMALL})
+      n = std::max<long>(n, tiling2(c->nt, L, pred, e[0] - 2, e[1] - 2).blocks());
+  }
   return n;
 }
 

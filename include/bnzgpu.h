@@ -170,9 +170,9 @@ int bnz_save_state(bnz_ctx *ctx, void *host, long bytes);
 int bnz_load_state(bnz_ctx *ctx, const void *host, long bytes);
 
 /* 0, 0, 0 (the default): 2D grids and large 3D grids run each stage of the
-   VL step as one fused pass (fluxes, EMFs and update; characteristic
-   limiting, the upwind EMF and user boundaries excepted).  Any other setting
-   runs the separate kernels.
+   VL step as one fused pass (fluxes, EMFs and update) where their shape makes
+   that the faster way; thin grids, characteristic limiting, the upwind EMF and
+   user boundaries keep the separate kernels.  Any other setting runs those.
    Work shapes of the separate 3D Godunov-flux, edge-EMF and stage-update
    kernels:
    0 one thread per face/edge/cell in x-fastest order (the

@@ -170,3 +170,43 @@ def test_ghosts_of_the_shortest_walled_axis(n, axis, hi, prec):
         last = f[5] if hi == 1 else 0.0 * f[5]
         assert np.array_equal(f[0], -last)
         assert np.abs(f[5][tuple(other)]).min() > 0.0
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32c"])
+@pytest.mark.parametrize("n,fused", [
+    ((128, 128, 128), "both"), ((98, 98, 98), "both"), ((96, 96, 96), "fp64"),
+    ((5, 320, 300), "fp64"), ((72, 72, 72), ""),
+    ((1000, 3, 200), ""), ((400, 400, 4), "both"), ((3, 30000, 1), "fp64"),
+    ((30000, 3, 1), "both"), ((3, 900, 1), "both")])
+def test_thin_grids_keep_the_separate_kernels(n, fused, prec):
+    """Tiles and columns run where they are the faster route."""
+    from bonzo_amd._lib import Context
+    print(f"case: {n} {prec}", flush=True)
+    s, prim, bfld = _state(*n, 3, 61)
+    out = []
+    for tune in ((0, 0, 0), (0, 1, 1)):
+        g = Context(*n, precision=prec)
+        g.set_tuning(*tune)
+        g.upload(prim, bfld)
+        g.init_state()
+        g.set_kernel_timing(True)
+        g.run_steps(2)
+        g.set_kernel_timing(False)
+        names = set(g.kernel_timing())
+        stage = any(name.startswith("stage") for name in names)
+        assert stage == (fused in ("both", prec) and tune == (0, 0, 0)), names
+        assert stage != any(name.startswith("flux") for name in names), names
+        out.append(g.download())
+        g.close()
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32c"])
+@pytest.mark.parametrize("nx,ny", [(11111, 12), (8, 14285), (12, 9000)])
+def test_tiles_of_long_thin_grids(nx, ny, prec):
+    print(f"case: {nx}x{ny} {prec}", flush=True)
+    s, prim, bfld = _state(nx, ny, 1, 3, 62)
+    a = _run(s, prim, bfld, 2, precision=prec)
+    b = _run(s, prim, bfld, 2, tune=(0, 1, 0), precision=prec)
+    _same(a, b, prec)
