@@ -481,6 +481,24 @@ void axis_coords(int N, int ind1, int ind2, int nact, double lmin, double lmax, 
   }
 }
 
+// FP32C 2D boxes that run separate kernels where there are many: thin ones, of
+// which tiles waste more than they save.  threads: those of the better tile's
+// stages a cell, the corrector's, which cost twice the predictor's, counted
+// twice.  us per step of 64 boxes of 1e6 cells together, separate / tiles,
+// (threads): 3x1736 209 / 273 (2.4), 4x1562 208 / 251 (2.1), 12x868 206 / 222 (2.0),
+// 5x1420 210 / 233 (1.94), 9x1041 207 / 204 (1.9), 10x976 207 / 187 (1.8), 15x744
+// 204 / 210 (1.7), 1736x3 168 / 177 (1.9), 976x10 167 / 158 (1.6).  FP64 boxes:
+// 3x1736 313 / 331, 12x868 312 / 320, all others faster with tiles.
+constexpr long THIN2_CELLS32 = 1L << 17;
+bool thin_box32(const BoxDev &d) {
+  if (d.g.dims != 2) return false;
+  const auto threads = [&](const int *e) {
+    return tile_threads(d.g.nt, d.L[0], true, e) + 2 * tile_threads(d.g.nt, d.L[1], false, e);
+  };
+  return std::min(threads(TILE2_SMALL), threads(TILE2_BIG32)) >
+         1.85 * 3. * (double)d.g.nt[0] * d.g.nt[1];
+}
+
 Box mkbox(int i0, int ni, int j0, int nj, int k0, int nk) {
   Box b;
   b.lo[0] = i0; b.n[0] = ni;
@@ -538,7 +556,7 @@ void b_stages(bnz_batch *c) {
 // stage updates of the 3D boxes, then the fused stages of the others
 template <bool PRED>
 void b_update(bnz_batch *c) {
-  const WList wl = wlist_dims(c, KUPD, 3);
+  const WList wl = wlist_dims(c, KSEP, 3);
   if (wl.hi != wl.lo)
     hipLaunchKernelGGL((kb_update<PRED>), dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(BLK), 0,
                        c->stream, c->boxes, wl, c->S, c->P, c->p.dt_fms_ref);
@@ -845,12 +863,6 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
       }
       if (dims < 2) L.lo[1] = L.hi[1] = 0;
       if (dims < 3) L.lo[2] = L.hi[2] = 0;
-      const int il = L.lo[0], iu = L.hi[0], jl = L.lo[1], ju = L.hi[1], kl = L.lo[2], ku = L.hi[2];
-      // 1D and 2D boxes keep their fluxes and EMFs in LDS: no items
-      const Box none = mkbox(0, 0, 0, 0, 0, 0);
-      d.items[o == 0 ? KF0 : KF1] = dims < 3 ? none : flux3_box(dims, L);
-      d.items[o == 0 ? KEM0 : KEM1] =
-          dims < 3 ? none : mkbox(il, iu + 2 - il, jl, ju + 2 - jl, kl, ku + 2 - kl);
     }
     d.items[KUPD] = mkbox(0, nt[0], 0, nt[1], 0, nt[2]);
     d.items[KS1] = dims == 1 ? mkbox(0, nt[0], 0, 1, 0, 1) : mkbox(0, 0, 0, 0, 0, 0);
@@ -872,10 +884,6 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
       d.bnd.flag[q] = s.bc[q];
       if (q < 2 * dims && s.bc[q] == BNZ_BC_REFLECT) d.bnd.plain = 0;
     }
-    if (dims == 2 || (all1 && !c->f32))
-      build_ghosts(nt, dims, ng, s.bc, off, pairs2, gops2);
-    else
-      build_ghosts(nt, dims, ng, s.bc, off, pairs, gops);
     off += (long)nt[0] * nt[1] * nt[2];
     if (off >= (1L << 31))
       return bfail(c, BNZ_EINVAL, "batch too large: pool cell indices are 32-bit");
@@ -883,28 +891,64 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   c->ncell = off;
   c->step1 = true;
   for (int b = 0; b < nbox; ++b) c->step1 = c->step1 && c->hbox[b].g.dims == 1;
+  // 2D boxes: tiles as the single grid's stages (tiling2), but for thin ones
+  long sep2 = 0;
+  for (const BoxDev &d : c->hbox)
+    if (c->f32 && thin_box32(d)) sep2 += (long)d.g.nt[0] * d.g.nt[1];
+  const bool sep = sep2 > THIN2_CELLS32;
+  const auto separate = [&](const BoxDev &d) {
+    return d.g.dims == 3 || (sep && thin_box32(d));
+  };
+  // together the boxes fill the chip, so the sum of their cells decides their
+  // tile's size, and the threads it takes
+  const int *big = c->f32 ? TILE2_BIG32 : TILE2_BIG64;
+  long cells2 = 0, small_threads = 0, big_threads = 0;
+  bool flux_pools = false;
+  for (int b = 0; b < nbox; ++b) {
+    const BoxDev &d = c->hbox[b];
+    flux_pools = flux_pools || d.g.dims == 1 || separate(d);
+    if (separate(d) || (d.g.dims == 1 && !(all1 && !c->f32)))
+      build_ghosts(d.g.nt, d.g.dims, ng, boxes[b].bc, d.off, pairs, gops);
+    else
+      build_ghosts(d.g.nt, d.g.dims, ng, boxes[b].bc, d.off, pairs2, gops2);
+    if (d.g.dims != 2 || separate(d)) continue;
+    cells2 += (long)d.g.nt[0] * d.g.nt[1];
+    for (int o = 0; o < 2; ++o) {
+      small_threads += tile_threads(d.g.nt, d.L[o], o == 0, TILE2_SMALL);
+      big_threads += tile_threads(d.g.nt, d.L[o], o == 0, big);
+    }
+  }
   c->nghost_step = (long)pairs.size();
   c->ngops_step = (long)gops.size();
   pairs.insert(pairs.end(), pairs2.begin(), pairs2.end());
   gops.insert(gops.end(), gops2.begin(), gops2.end());
   c->nghost = (long)pairs.size();
   c->ngops = (long)gops.size();
-  // tiles of the 2D boxes, as the single grid's stages (tiling2): together
-  // the boxes fill the chip, so the sum of their cells decides their size
-  long cells2 = 0;
-  bool any[4] = {};
-  for (const BoxDev &d : c->hbox) {
-    any[d.g.dims] = true;
-    if (d.g.dims == 2) cells2 += (long)d.g.nt[0] * d.g.nt[1];
-  }
-  c->tile_small = cells2 <= TILE2_SMALL_CELLS;
-  for (BoxDev &d : c->hbox)
+  // us per step of 64 boxes, small / big tile: FP64 1736x3 263 / 303, 1562x4 250
+  // / 270, 744x15 248 / 260 (the same threads), 1302x6 239 / 242, 36x372 242 / 217
+  // (a sixth more); FP32C 10x976 187 / 245, 30x434 191 / 231, 36x372 170 / 196,
+  // 1562x4 160 / 169 (a sixth more), 60x236 177 / 195 (0.94), 372x36 164 / 147
+  c->tile_small = cells2 <= TILE2_SMALL_CELLS ||
+                  (c->f32 ? 10 * small_threads <= 9 * big_threads : small_threads <= big_threads);
+  const int *e = c->tile_small ? TILE2_SMALL : big;
+  for (BoxDev &d : c->hbox) {
+    const Box none = mkbox(0, 0, 0, 0, 0, 0);
+    const int *nt = d.g.nt;
     for (int o = 0; o < 2; ++o) {
-      const int *e = c->tile_small ? TILE2_SMALL : c->f32 ? TILE2_BIG32 : TILE2_BIG64;
-      const Tiling t = tiling2(d.g.nt, d.L[o], o == 0, e[0] - 2, e[1] - 2);
-      d.items[o == 0 ? KP2 : KC2] = d.g.dims == 2 ? mkbox(t.o[0], t.n[0], t.o[1], t.n[1], 0, 1)
-                                                  : mkbox(0, 0, 0, 0, 0, 0);
+      const Lims &L = d.L[o];
+      const Tiling t = tiling2(nt, L, o == 0, e[0] - 2, e[1] - 2);
+      const int nk = d.g.dims == 3 ? L.hi[2] + 2 - L.lo[2] : 1;
+      d.items[o == 0 ? KF0 : KF1] = separate(d) ? flux3_box(d.g.dims, L) : none;
+      d.items[o == 0 ? KEM0 : KEM1] =
+          separate(d) ? mkbox(L.lo[0], L.hi[0] + 2 - L.lo[0], L.lo[1], L.hi[1] + 2 - L.lo[1],
+                              L.lo[2], nk)
+                      : none;
+      d.items[o == 0 ? KP2 : KC2] = d.g.dims == 2 && !separate(d)
+                                        ? mkbox(t.o[0], t.n[0], t.o[1], t.n[1], 0, 1)
+                                        : none;
     }
+    d.items[KSEP] = separate(d) ? d.items[KUPD] : none;
+  }
   // work blocks: box b owns ceil(items / BLK) consecutive blocks of each
   // list; the 1D boxes come first, then the 2D and the 3D boxes
   std::vector<int> hmap;
@@ -939,7 +983,7 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
               {&c->P.fy, NMODE}, {&c->P.fz, NMODE}};
   // FP32C keeps prim (upload, download) and the faces in FP64; its work
   // arrays are the FP32 pools below
-  const int nflux = any[1] || any[3] ? 3 : 0;  // the 2D stages have no flux arrays
+  const int nflux = flux_pools ? 3 : 0;  // the 2D stages have no flux arrays
   const int nb64 = c->f32 ? 3 : 5 + nflux;
   for (int q = 0; q < nb64; ++q) {
     if (hipMalloc(bufs[q].q, bufs[q].rows * cells * sizeof(double)) != hipSuccess)

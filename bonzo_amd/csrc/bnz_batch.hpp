@@ -12,13 +12,14 @@ namespace bnzb {
 using namespace bnz;
 
 // work lists: fluxes (all directions, one item per cell of the union of the
-// face ranges) and EMFs of the predictor and of the corrector of the 3D
-// boxes, all cells (3D stage updates, copies), active cells (init and the
-// first CFL maximum), the cells of the 1D boxes for the fused 1D stage (BLK - 1
+// face ranges) and EMFs of the predictor and of the corrector of the boxes
+// that run separate kernels (3D, and thin 2D ones in FP32C), all cells
+// (copies), active cells (init and the first CFL maximum), the cells of the 1D boxes for the fused 1D stage (BLK - 1
 // per work block) and for the fused 1D step of all-1D batches (BLK - 6 per
-// work block), the tiles of the 2D boxes for the fused 2D stages (predictor
-// and corrector; a work block is a tile, items are tiles from the origin lo)
-enum { KF0 = 0, KEM0, KF1, KEM1, KUPD, KACT, KS1, KT1, KP2, KC2, NK };
+// work block), the tiles of the other 2D boxes for the fused 2D stages
+// (predictor and corrector; a work block is a tile, items are tiles from the
+// origin lo), and all cells of the boxes with separate kernels (their updates)
+enum { KF0 = 0, KEM0, KF1, KEM1, KUPD, KACT, KS1, KT1, KP2, KC2, KSEP, NK };
 
 // items per work block of list kt
 __host__ __device__ constexpr int blk_items(int kt) {

@@ -22,8 +22,9 @@ __device__ __forceinline__ Walls box_walls(const BoxDev &d) {
   return wl;
 }
 
-// The flux, EMF and update kernels of the 3D boxes.
-template <int ORDER, int RS, typename BF>
+// The flux, EMF and update kernels of the boxes that run separate kernels,
+// compiled per dimensionality.
+template <int ORDER, int RS, typename BF, int DIMS>
 __global__ __launch_bounds__(BLK) void kb32_flux(const BoxDev *__restrict__ boxes, WList wl,
                                                  BoxState st, const float *__restrict__ w,
                                                  const BF *__restrict__ bf,
@@ -40,12 +41,13 @@ __global__ __launch_bounds__(BLK) void kb32_flux(const BoxDev *__restrict__ boxe
     int i, j, k;
     box_idx(it, t, i, j, k);
     const long o = d.off;
-    flux32_cell<ORDER, RS, BF, 3>(d.g, w + o, bf + o, fx + o, fy + o, fz + o,
+    flux32_cell<ORDER, RS, BF, DIMS>(d.g, w + o, bf + o, fx + o, fy + o, fz + o,
                                      d.L[wl.kt == KF0 ? 0 : 1], i, j, k, ng);
   }
   if (ng) atomicAdd(nguard, ng);
 }
 
+template <int DIMS>
 __global__ __launch_bounds__(BLK) void kb32_emf(const BoxDev *__restrict__ boxes, WList wl,
                                                 BoxState st, const float *__restrict__ w,
                                                 const float *__restrict__ fx,
@@ -62,14 +64,14 @@ __global__ __launch_bounds__(BLK) void kb32_emf(const BoxDev *__restrict__ boxes
     int i, j, k;
     box_idx(it, t, i, j, k);
     const long o = d.off;
-    emf32_edge<3>(d.g, w + o, fx + o, fy + o, fz + o, ee + o, box_walls(d), i, j, k);
+    emf32_edge<DIMS>(d.g, w + o, fx + o, fy + o, fz + o, ee + o, box_walls(d), i, j, k);
   }
 }
 
 // Stage update of every cell of the running boxes (update32_pred /
 // update32_corr); the corrector folds the CFL maximum into the box's cmax.
 // A finished box is left alone (its faces: BoxState::fpar, kb_face_fix).
-template <bool PRED>
+template <bool PRED, int DIMS>
 __global__ __launch_bounds__(BLK) void kb32_update(const BoxDev *__restrict__ boxes, WList wl,
                                                    BoxState st, Pools P, Pools32 Q,
                                                    int fms_ref) {
@@ -87,11 +89,11 @@ __global__ __launch_bounds__(BLK) void kb32_update(const BoxDev *__restrict__ bo
       if (PRED) {
         const Pred32 a{Q.w32 + o, Q.uh + o, P.b + o, Q.fx + o, Q.fy + o,
                        Q.fz + o,  Q.ee + o, Q.bs32 + o, Q.ws32 + o};
-        update32_pred<3>(d.g, a, d.L[0], st.dt + b, i, j, k);
+        update32_pred<DIMS>(d.g, a, d.L[0], st.dt + b, i, j, k);
       } else {
         const Corr32 a{Q.uh + o, Q.ul + o, P.b + o, Q.fx + o, Q.fy + o,
                        Q.fz + o, Q.ee + o, P.bs + o, Q.w32 + o};
-        cds = update32_corr<3>(d.g, a, d.L[1], st.dt + b, d.act, fms_ref, i, j, k);
+        cds = update32_corr<DIMS>(d.g, a, d.L[1], st.dt + b, d.act, fms_ref, i, j, k);
       }
     }
     if (!PRED) block_max_atomic(cds, st.cmax + b);
@@ -334,14 +336,20 @@ __global__ __launch_bounds__(BLK) void kb32_ghost_ops(Ghost32 p, const GhostOp *
     ghost32_op(p, ops[t]);
 }
 
-// fluxes of the 3D boxes
+// fluxes of the boxes with separate kernels
 template <int ORDER, int RS, typename BF>
 void flux_launch(bnz_batch *c, const float *w, const BF *bf, int kt) {
-  const WList wl = wlist(c, kt);
-  if (wl.hi == wl.lo) return;
-  hipLaunchKernelGGL((kb32_flux<ORDER, RS, BF>), dim3(grid_for(wl.hi - wl.lo, c->cap[TF])),
-                     dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w, bf, c->Q.fx, c->Q.fy,
-                     c->Q.fz, c->nguard);
+  for (int d = 2; d <= 3; ++d) {
+    const WList wl = wlist_dims(c, kt, d);
+    if (wl.hi == wl.lo) continue;
+    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TF]));
+    if (d == 2)
+      hipLaunchKernelGGL((kb32_flux<ORDER, RS, BF, 2>), grid, dim3(BLK), 0, c->stream, c->boxes,
+                         wl, c->S, w, bf, c->Q.fx, c->Q.fy, c->Q.fz, c->nguard);
+    else
+      hipLaunchKernelGGL((kb32_flux<ORDER, RS, BF, 3>), grid, dim3(BLK), 0, c->stream, c->boxes,
+                         wl, c->S, w, bf, c->Q.fx, c->Q.fy, c->Q.fz, c->nguard);
+  }
 }
 
 template <typename BF>
@@ -356,12 +364,19 @@ void fluxes(bnz_batch *c, int order, const float *w, const BF *bf, int kt) {
   }
 }
 
-// EMFs of the 3D boxes
+// EMFs of the boxes with separate kernels
 void emfs(bnz_batch *c, const float *w, int kt) {
-  const WList wl = wlist(c, kt);
-  if (wl.hi == wl.lo) return;
-  hipLaunchKernelGGL(kb32_emf, dim3(grid_for(wl.hi - wl.lo, c->cap[TE])), dim3(BLK), 0, c->stream,
-                     c->boxes, wl, c->S, w, c->Q.fx, c->Q.fy, c->Q.fz, c->Q.ee);
+  for (int d = 2; d <= 3; ++d) {
+    const WList wl = wlist_dims(c, kt, d);
+    if (wl.hi == wl.lo) continue;
+    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TE]));
+    if (d == 2)
+      hipLaunchKernelGGL(kb32_emf<2>, grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w,
+                         c->Q.fx, c->Q.fy, c->Q.fz, c->Q.ee);
+    else
+      hipLaunchKernelGGL(kb32_emf<3>, grid, dim3(BLK), 0, c->stream, c->boxes, wl, c->S, w,
+                         c->Q.fx, c->Q.fy, c->Q.fz, c->Q.ee);
+  }
 }
 
 // the fused stages of the 1D and of the 2D boxes
@@ -391,13 +406,21 @@ void stages(bnz_batch *c) {
   stage1<PRED, ORDER, RS>(c);
 }
 
-// stage updates of the 3D boxes, then the fused stages of the others
+// stage updates of the boxes with separate kernels, then the fused stages of
+// the others
 template <bool PRED>
 void updates(bnz_batch *c) {
-  const WList wl = wlist_dims(c, KUPD, 3);
-  if (wl.hi != wl.lo)
-    hipLaunchKernelGGL((kb32_update<PRED>), dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(BLK),
-                       0, c->stream, c->boxes, wl, c->S, c->P, c->Q, c->p.dt_fms_ref);
+  for (int d = 2; d <= 3; ++d) {
+    const WList wl = wlist_dims(c, KSEP, d);
+    if (wl.hi == wl.lo) continue;
+    const dim3 grid(grid_for(wl.hi - wl.lo, c->cap[TU]));
+    if (d == 2)
+      hipLaunchKernelGGL((kb32_update<PRED, 2>), grid, dim3(BLK), 0, c->stream, c->boxes, wl,
+                         c->S, c->P, c->Q, c->p.dt_fms_ref);
+    else
+      hipLaunchKernelGGL((kb32_update<PRED, 3>), grid, dim3(BLK), 0, c->stream, c->boxes, wl,
+                         c->S, c->P, c->Q, c->p.dt_fms_ref);
+  }
   const bool hlld = c->p.rsolver == BNZ_RS_HLLD;
   if (PRED || c->order == 0) {
     if (hlld) stages<PRED, 0, BNZ_RS_HLLD>(c);

@@ -30,3 +30,25 @@ def test_batch_2d_stages_bitwise_vs_single(sizes, precision, rsolver, reconstr, 
         cases.insert(1, (P.riemann_tube(90, rng, ng=ng), (1,) * 6, 0.01))
         cases.append((_state(17, 9, 12, ng, 72), (2, 1, 0, 0, 1, 2), 0.005))
     check_against_single(cases, rsolver, reconstr, precision=precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("n,extra", [((3, 900), False), ((3, 900), True), ((900, 3), False),
+                                     ((12, 500), True), ((10, 600), False)])
+def test_thin_boxes(n, extra, precision):
+    """Many thin boxes: in FP32C some run separate kernels, beside boxes of
+    every other kind, in FP64 the tile goes by the threads it takes."""
+    say(f"case: 20 boxes of {n}, extra {extra}, {precision}")
+    cases = []
+    for q in range(20):
+        bc = SIDES[q % 4]
+        s, prim, bfld = _state(n[0], n[1] + q, 1, 3, 200 + q)
+        for a in (0, 1):
+            if 2 in bc[2 * a:2 * a + 2]:
+                bfld[a][:] = 0.0  # no field through a wall
+        cases.append(((s, prim, bfld), bc, (4e-4, 1e-4, 3e-4)[q % 3]))
+    if extra:
+        cases[3:3] = [(_state(70, 60, 1, 3, 231), (0,) * 6, 1e-3),
+                      (_state(90, 1, 1, 3, 232), (1,) * 6, 1e-3),
+                      (_state(12, 11, 10, 3, 233), (0,) * 6, 1e-3)]
+    check_against_single(cases, precision=precision)
