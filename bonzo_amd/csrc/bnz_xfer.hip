@@ -10,16 +10,21 @@
 namespace bnz {
 namespace {
 
-// The pinned buffer: one chunk per worker of a large transfer.  Chunks of 2 MB
-// are 37 us of bus time each, against about 5 us between launches.
+// The large pinned buffer: one chunk per worker of a large transfer.  Chunks of
+// 2 MB are 37 us of bus time each, against about 5 us between launches.
 constexpr int WORKERS = 8;
 constexpr size_t CHUNK = 2u << 20, CAP = WORKERS * CHUNK;
 constexpr long CHUNK_LEN = CHUNK / sizeof(double);
+// The small one: up to 1 MB the runtime hands out pinned memory in 15 to 70 us,
+// beyond in 300 to 900, and the first touch of its pages takes 0.4 us a KB.
+constexpr size_t SMALL = 1u << 20;
 // Below this plain arrays go through the runtime: two arrays of 50 KB take it
-// 50 us up and 60 down, and the pinned buffer is 80 us to set up.
+// 30 us up and 50 down.
 constexpr size_t DIRECT = 64u << 10;
 // From here on threads pay (starting one is some 20 us; one thread copies to
-// new pages at 10 GB/s, to old ones at 40).
+// new pages at 10 GB/s, to old ones at 40).  Four uploads and downloads of new
+// arrays, a process's first, by the runtime -> so: 1.2 MB 4.7 -> 2.4 ms, 4.2 MB
+// 12.8 -> 6.9, 19 MB 20.3 -> 7.8; 1 MB 3.9 -> 1.7 (2.3 with the large buffer).
 constexpr size_t THREADED = 2 * CHUNK;
 constexpr int BLOCK = 256, MAX_BLOCKS = 256;
 
@@ -93,14 +98,26 @@ HostLink::~HostLink() {
     if (e) (void)hipEventDestroy(e);
 }
 
-bool HostLink::reserve() {
-  if (pin_ || no_pin_) return pin_ != nullptr;
-  if (hipHostMalloc((void **)&pin_, CAP, hipHostMallocDefault) != hipSuccess) {
+// A pinned buffer for a transfer of so many bytes; cap_ stays too small where
+// there is no memory for one.
+hipError_t HostLink::reserve(hipStream_t stream, size_t bytes) {
+  if (no_pin_ || bytes <= cap_ || cap_ == CAP) return hipSuccess;
+  const size_t cap = bytes > SMALL ? CAP : SMALL;
+  if (pin_) {  // uploads in flight may still read the old one
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return e;
+    (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    cap_ = used_ = 0;
+  }
+  if (hipHostMalloc((void **)&pin_, cap, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     pin_ = nullptr;
+  } else {
+    cap_ = cap;
   }
   no_pin_ = pin_ == nullptr;
-  return pin_ != nullptr;
+  return hipSuccess;
 }
 
 // Without pinned memory: row by row through the runtime.
@@ -124,10 +141,13 @@ hipError_t HostLink::move(int device, hipStream_t stream, const Seg *s, int n, b
   const long total = s[0].total() + (n > 1 ? s[1].total() : 0);
   const size_t bytes = total * sizeof(double);
   const bool plain = s[0].rows == 1 && (n < 2 || s[1].rows == 1);
-  if ((plain && bytes < DIRECT) || !reserve()) return direct(stream, s, n, to_dev);
+  if (plain && bytes < DIRECT) return direct(stream, s, n, to_dev);
+  hipError_t e0 = reserve(stream, bytes);
+  if (e0 != hipSuccess) return e0;
+  if (cap_ < std::min(bytes, CAP)) return direct(stream, s, n, to_dev);
   if (bytes < THREADED) {
     hipError_t e = hipSuccess;
-    if (used_ + bytes > CAP) {
+    if (used_ + bytes > cap_) {
       if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
       used_ = 0;
     }
@@ -145,8 +165,7 @@ hipError_t HostLink::move(int device, hipStream_t stream, const Seg *s, int n, b
   }
   // Large: each worker owns a chunk of the buffer and takes the next piece of
   // the arrays when it is free, so the workers need no word with each other.
-  hipError_t e0 = hipStreamSynchronize(stream);
-  if (e0 != hipSuccess) return e0;
+  if ((e0 = hipStreamSynchronize(stream)) != hipSuccess) return e0;
   used_ = 0;
   for (hipEvent_t &e : ev_)
     if (!e && (e0 = hipEventCreateWithFlags(&e, hipEventDisableTiming)) != hipSuccess) return e0;

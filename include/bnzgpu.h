@@ -118,7 +118,11 @@ int bnz_get_shape(const bnz_ctx *ctx, int *ntot3, int *ng);
 
 /* Host <-> device copies of the grid arrays (GridData, grid.pyx:28-52).
    upload waits for the context's queued work; the state then needs
-   bnz_init_state (or bnz_load_state) before the next step. */
+   bnz_init_state (or bnz_load_state) before the next step.  A context whose
+   transfers take 64 KB or more, and a batch from its first box on, hold
+   pinned host memory for them until they are destroyed: 1 MB, or 16 MB once
+   a transfer was larger than that; without any, transfers go through the
+   runtime. */
 int bnz_upload(bnz_ctx *ctx, const double *prim, const double *bfld);
 int bnz_download(bnz_ctx *ctx, double *prim, double *bfld, double *cons);
 
