@@ -108,6 +108,15 @@ int main() {
       CHECK(a.host == std::vector<double>(len, 42.));
     }
   }
+  {  // small downloads: a wait and blocking copies, which cost less than two
+     // asynchronous ones and a wait
+    FakeStream st;
+    HostLink link;
+    Arrays a(1, 90, 90, 3.), b(1, 30, 30, 4.);
+    const Seg s[2] = {a.seg(), b.seg()};
+    const long before = st.issued;
+    CHECK(link.down(0, &st, s, 2) == hipSuccess && st.issued == before);
+  }
   printf("%d failures\n", bad);
   return bad ? 1 : 0;
 }
