@@ -4,7 +4,6 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
 #include <thread>
 
 namespace bnz {
@@ -203,8 +202,8 @@ hipError_t HostLink::move(int device, hipStream_t stream, const Seg *s, int n, b
   for (int w = 1; w < workers; ++w) {
     try {
       pool[w] = std::thread(work, w);
-    } catch (const std::system_error &) {
-      break;  // no more threads: the others take the pieces
+    } catch (...) {
+      break;  // no more threads or memory: the others take the pieces
     }
   }
   work(0);

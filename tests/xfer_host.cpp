@@ -1,11 +1,22 @@
 // The transfers of bnz_xfer.hip (HostLink) on a stand-in runtime whose stream
 // runs late: every route, what each pins, and what the caller may reuse when.
 #include <cstdio>
+#include <new>
 #include <vector>
 
 #include "../bonzo_amd/csrc/bnz_xfer.hip"
 
 using namespace bnz;
+
+// the n-th allocation of this thread fails
+static thread_local int fail_new = 0;
+void *operator new(size_t n) {
+  if (fail_new && --fail_new == 0) throw std::bad_alloc();
+  if (void *p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 static int bad = 0;
 #define CHECK(x) \
@@ -116,6 +127,22 @@ int main() {
     const Seg s[2] = {a.seg(), b.seg()};
     const long before = st.issued;
     CHECK(link.down(0, &st, s, 2) == hipSuccess && st.issued == before);
+  }
+  {  // no memory to start the threads with: the caller's moves everything
+    FakeStream st;
+    HostLink link;
+    Arrays a(1, 3000000, 3000000, 6.);
+    const Seg s = a.seg();
+    CHECK(link.up(0, &st, &s, 1) == hipSuccess);
+    std::fill(a.pool.begin(), a.pool.end(), 0.);
+    try {
+      fail_new = 1;  // a second call's first allocation is its first thread's
+      CHECK(link.up(0, &st, &s, 1) == hipSuccess && fail_new == 0);
+    } catch (...) {
+      CHECK(!"no exception leaves a transfer");
+    }
+    fail_new = 0;
+    CHECK(a.up_ok(6.));
   }
   printf("%d failures\n", bad);
   return bad ? 1 : 0;
