@@ -188,8 +188,12 @@ int bnz_load_state(bnz_ctx *ctx, const void *host, long bytes);
    places the edge EMFs of the separate kernels instead: 0 forms them inside the
    update launches up to 2^18 cells with ghosts and in launches of their own
    beyond, 1 always in launches of their own, 2 or more always inside the
-   updates.  Results do not depend on either choice.  Chosen by the
-   autotuner (bonzo_amd/autotune.py, 3D); no counterpart in the reference. */
+   updates.  Results do not depend on any of this, but for a face whose solver
+   matches no region (speeds that are not numbers: negative pressure or
+   density, states that are not finite; bnz_diag tells): its flux is 0 in a
+   fused stage, as in the first stages of a new context, and keeps its row in
+   the separate kernels, as in the reference.  Chosen by the autotuner
+   (bonzo_amd/autotune.py, 3D); no counterpart in the reference. */
 int bnz_set_tuning(bnz_ctx *ctx, int flux_chunk, int emf_chunk, int update_chunk);
 
 /* User boundary (flag 3) of one side.  The reference leaves such a side's

@@ -210,3 +210,32 @@ def test_tiles_of_long_thin_grids(nx, ny, prec):
     a = _run(s, prim, bfld, 2, precision=prec)
     b = _run(s, prim, bfld, 2, tune=(0, 1, 0), precision=prec)
     _same(a, b, prec)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32c"])
+@pytest.mark.parametrize("n", [(150, 140, 1), (104, 98, 112)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -1.0])
+def test_a_bad_cell_stays_where_it_is(n, value, prec):
+    """A cell that is not finite, or of negative density: a face whose solver
+    matches no region has flux 0 in a fused stage.  Cells that a step's stages
+    do not reach from it are the separate kernels' bit for bit, and finite."""
+    from bonzo_amd._lib import Context
+    print(f"case: {n} {value} {prec}", flush=True)
+    s, prim, bfld = _state(*n, 3, 63)
+    at = [3 + m // 2 if m > 1 else 0 for m in n]
+    prim[0][at[2], at[1], at[0]] = value
+    out = []
+    for tune in ((0, 0, 0), (0, 0, 1) if n[2] > 1 else (0, 1, 0)):
+        g = Context(*n, precision=prec)
+        g.set_tuning(*tune)
+        g.upload(prim, bfld)
+        g.init_state()
+        assert g.diag()["bad_ijk"] == tuple(at)
+        g.vl_step(1e-4)
+        out.append(g.download())
+        g.close()
+    far = np.ones(prim.shape[1:], bool)  # outside the cells the two stages reach
+    far[tuple(slice(max(0, x - 6), x + 7) for x in reversed(at))] = False
+    for x, y in zip(*out):
+        assert np.isfinite(x[:, far]).all()
+        assert np.array_equal(x[:, far], y[:, far])
