@@ -239,3 +239,24 @@ def test_a_bad_cell_stays_where_it_is(n, value, prec):
     for x, y in zip(*out):
         assert np.isfinite(x[:, far]).all()
         assert np.array_equal(x[:, far], y[:, far])
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32c"])
+def test_columns_beyond_256_cubed(prec):
+    """Columns against the separate kernels on a grid larger than any other here,
+    of sides that end inside a tile and a run of planes."""
+    n = (272, 261, 285)
+    print(f"case: {n} {prec}", flush=True)
+    s, prim, bfld = _state(8, 9, 10, 3, 64)  # a small state, repeated over the grid
+    big = P.GridShape(*n, 3)
+    w, b = big.empty()
+    act = big.active()
+    for dst, src in ((w, prim), (b, bfld)):
+        for v in range(dst.shape[0]):
+            tile = src[v][s.active()]
+            reps = [-(-m // t) for m, t in zip(reversed(n), tile.shape)]
+            dst[v][act] = np.tile(tile, reps)[:n[2], :n[1], :n[0]]
+    bc = (0, 0, 1, 2, 0, 0)
+    a = _run(big, w, b, 1, bc=bc, precision=prec)
+    c = _run(big, w, b, 1, tune=(0, 0, 1), bc=bc, precision=prec)
+    _same(a, c, prec)

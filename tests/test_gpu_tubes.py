@@ -156,3 +156,50 @@ def test_one_launch_steps_against_the_oracle(nx, precision, char_proj):
         assert g.advance(t + 0.4 * dt) == 1 and g.time()[0] == t + 0.4 * dt
     g.close()
     o.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp64fma"])
+@pytest.mark.parametrize("nx", [744, 745, 743, 994])
+def test_one_launch_steps_at_the_ends_of_workgroups(nx, precision):
+    """Grids whose last workgroup (250 cells each, ghosts included) is just full,
+    holds one cell, lacks one, or is full again: IEEE bit for bit, FMA to 1e-12
+    relative L1."""
+    from bonzo_amd._lib import Context
+    from oracle.oracle import OracleSim
+    bc = SIDES[nx % 5]
+    print(f"case: {nx} {precision} bc {bc}", flush=True)
+    s, prim, bfld = _state(nx, 1, 1, 3, 140 + nx)
+    bfld[0][:] = 0.0 if 2 in bc else 0.3
+    o = OracleSim(nx, bc=bc)
+    o.prim[:] = prim
+    o.bfld[:] = bfld
+    o.init()
+    o.advance_steps(7)
+    g = Context(nx, bc=bc, precision=precision)
+    g.upload(prim, bfld)
+    g.init_state()
+    g.run_steps(7)
+    gp, gb = g.download()
+    g.close()
+    for x, y in ((gp, o.prim), (gb, o.bfld)):
+        x, y = x[..., 3:-3], y[..., 3:-3]
+        if precision == "fp64":
+            assert np.array_equal(x, y)
+        else:
+            for v in range(x.shape[0]):
+                den = max(np.abs(y[v]).sum(), 1e-9 * np.abs(prim[0]).sum())
+                assert np.abs(x[v] - y[v]).sum() <= 1e-12 * den, v
+    o.close()
+
+
+@pytest.mark.parametrize("reconstr", ["linear", "const"])
+def test_batch_steps_at_the_ends_of_workgroups(reconstr):
+    say(f"case: boxes of 744, 745, 743, 994 cells {reconstr}")
+    ng = 2 if reconstr == "const" else 3
+    cases = []
+    for q, n in enumerate((744, 745, 743, 994)):
+        s, prim, bfld = _state(n + 6 - 2 * ng, 1, 1, ng, 150 + q)
+        bc = SIDES[q % 5]
+        bfld[0][:] = 0.0 if 2 in bc else 0.3  # no field through a wall
+        cases.append(((s, prim, bfld), bc, 0.004))
+    check_against_single(cases, "hlld", reconstr)
