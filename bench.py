@@ -54,13 +54,17 @@ KERNEL_BYTES = {
 # sampled SIMDs' cycles spent issuing VALU work (SQ_ACTIVE_INST_VALU x 4 /
 # (GRBM_GUI_ACTIVE x SIMDs); near 1 a launch is bound by arithmetic issue),
 # from the rocprofv3 --pmc runs summarised in the named profile, per work
-# shape of the kernel's class (0 flat, n > 1 slab columns of n rows; the
-# FP32C tile shape runs flat); the bench itself runs no counters.  FETCH_SIZE
+# shape of the kernel's class (0 flat or fused, n > 1 slab columns of n rows;
+# the FP32C tile shape runs flat); the bench itself runs no counters.  FETCH_SIZE
 # counts reads that the MALL serves too, which the flat launches (workgroups
 # in runs dealt round-robin over the XCDs) lean on, so for them it bounds the
 # HBM bytes from above.
 PROFILE = "profiles/vl_step_kernels_turb256.md"
+PROFILE_STAGES = "profiles/fused_stage_kernels.md"
 PROFILED = {
+    ("fp64fma", "stage_corr", 0): (9.013e9, 0.73),
+    ("fp64", "stage_corr", 0): (8.952e9, 0.79),
+    ("fp32c", "stage_corr", 0): (8.265e9, 0.76),
     ("fp64fma", "flux3_plm", 0): (8.298e9, 0.64),
     ("fp64fma", "flux3_plm", 8): (5.995e9, 0.58),
     ("fp64", "flux3_plm", 0): (8.298e9, 0.76),
@@ -222,12 +226,15 @@ def run_path(prec, n, prim, bfld, args):
     b = kernel_bytes(prec, dname, n)
     ach = b / (davg * 1e-3) / 1e9
     traffic, busy = profiled(prec, dname, tuned) if n == 256 else (None, None)
+    source = PROFILE_STAGES if dname.startswith("stage") else PROFILE
+    # what binds it: arithmetic issue where that takes the larger share of its time
+    bound = "valu" if busy is not None and busy > ach / HBM_PEAK_GBS else "hbm"
     return {
         "value": value, "ms_per_step": 1e3 * el / args.steps, "tuned": tuned, "table": table,
         "kernels": {k: v[0] / v[1] for k, v in sorted(kt.items())},
-        "roofline": {"bound": "hbm", "kernel": dname, "achieved": ach, "peak": HBM_PEAK_GBS,
+        "roofline": {"bound": bound, "kernel": dname, "achieved": ach, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
-                     "traffic": traffic, "traffic_source": PROFILE if traffic else None,
+                     "traffic": traffic, "traffic_source": source if traffic else None,
                      "valu_busy": busy,
                      "avg_launch_ms": davg, "algorithmic_bytes_per_launch": b},
         "step_GBs": STEP_BYTES[prec] * value / 1e9,

@@ -875,15 +875,12 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
     }
     d.bnd.ng = ng;
     d.bnd.dims = dims;
-    d.bnd.plain = 1;
     for (int a = 0; a < 3; ++a) {
       d.bnd.a1[a] = a1[a];
       d.bnd.a2[a] = a2[a];
     }
-    for (int q = 0; q < 6; ++q) {
-      d.bnd.flag[q] = s.bc[q];
-      if (q < 2 * dims && s.bc[q] == BNZ_BC_REFLECT) d.bnd.plain = 0;
-    }
+    for (int q = 0; q < 6; ++q) d.bnd.flag[q] = s.bc[q];
+    d.bnd.close();
     off += (long)nt[0] * nt[1] * nt[2];
     if (off >= (1L << 31))
       return bfail(c, BNZ_EINVAL, "batch too large: pool cell indices are 32-bit");

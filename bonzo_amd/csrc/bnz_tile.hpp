@@ -168,20 +168,29 @@ struct ColGeo<true> {
 // The boundaries of a grid, for the kernels that write the ghost cells along
 // with the active cells they copy (build_ghosts composes per-axis maps, so
 // the ghosts of an active cell are the products of its images per axis).
+enum { END_NONE = 0, END_WALL = 1, END_FACE = 2 };  // END_FACE: the image's bit
 struct Bnd {
   int a1[3], a2[3];  // first and last active index
   int flag[6];       // BNZ_BC_PERIODIC, _OUTFLOW or _REFLECT per side
   int ng, dims;
   int plain;         // no reflecting side
+  int end[3];        // END_*, see close
+  // The low ghosts of an axis can mirror a face past its active cells: with a
+  // reflecting low side and just ng cells, ghost face a1 - ng mirrors face
+  // a2 + 1, which the high side sets.  It then mirrors what that side copies
+  // there: face a2 with outflow, else a wall face, 0 (build_ghosts does the
+  // same).  Worked out here, once, to keep the kernels short.
+  void close() {
+    plain = 1;
+    for (int a = 0; a < 3; ++a) {
+      end[a] = END_NONE;
+      if (a >= dims) continue;
+      if (flag[2 * a] == BNZ_BC_REFLECT || flag[2 * a + 1] == BNZ_BC_REFLECT) plain = 0;
+      if (flag[2 * a] == BNZ_BC_REFLECT && a2[a] - a1[a] + 1 == ng)
+        end[a] = flag[2 * a + 1] == BNZ_BC_OUTFLOW ? END_FACE : END_WALL;
+    }
+  }
 };
-
-// Whether the low ghosts of an axis mirror a face past its active cells: with a
-// reflecting low side and just ng cells, ghost face a1 - ng mirrors face
-// a2 + 1, which the high side sets.  It then mirrors what that side copies
-// there: face a2 with outflow, else a wall face, 0 (build_ghosts does the same).
-__host__ __device__ __forceinline__ bool low_mirrors_end(const Bnd &b, int axis) {
-  return b.flag[2 * axis] == BNZ_BC_REFLECT && b.a2[axis] - b.a1[axis] + 1 == b.ng;
-}
 
 // Images of index x along one axis, bit 0 x itself, bit 1 + g the low ghost
 // a1 - ng + g, bit 1 + ng + g the high ghost a2 + 1 + g.  FACE: the images of
@@ -200,7 +209,7 @@ __host__ __device__ __forceinline__ unsigned images(const Bnd &b, int axis, int 
   }
   if (hi == BNZ_BC_OUTFLOW) {
     if (x == a2) m |= ((1u << ng) - 1) << (1 + ng);
-    if (FACE && x == a2 && low_mirrors_end(b, axis)) m |= 2u;
+    if (FACE && x == a2) m |= b.end[axis];
   } else {
     const int q = hi == BNZ_BC_PERIODIC ? x + n : FACE ? 2 * a2 + 2 - x : 2 * a2 + 1 - x;
     const int q0 = (FACE && hi == BNZ_BC_REFLECT) ? a2 + 2 : a2 + 1;
@@ -269,32 +278,25 @@ __host__ __device__ __forceinline__ void scatter_ghosts(const Bnd &b, const Geo 
     }
     unsigned f[3] = {m[0], m[1], m[2]};
     f[a] = a == 0 ? images<true>(b, 0, i) : a == 1 ? images<true>(b, 1, j) : images<true>(b, 2, k);
-    const bool zlo = b.flag[2 * a] == BNZ_BC_REFLECT && x[a] == b.a1[a];
-    const bool zhi = b.flag[2 * a + 1] == BNZ_BC_REFLECT && x[a] == b.a2[a];
-    const bool zend = b.flag[2 * a + 1] != BNZ_BC_OUTFLOW && x[a] == b.a2[a] &&
-                      low_mirrors_end(b, a);
     each_image(b, g, f, i, j, k,
                [&](long dst, unsigned flips) { face(a, dst, ((flips >> a) & 1u) != 0); });
-    if (zlo || zhi || zend) {
-      // the wall face itself (zend: its mirror image past the low ghosts) and
-      // its images along the other axes
-      unsigned o[3] = {m[0], m[1], m[2]};
-      o[a] = 1u;
-      const long step = a == 0 ? 1 : a == 1 ? g.sy : g.sz;
-      const long self = ((long)k * g.nt[1] + j) * g.nt[0] + i;
-      if (zlo) {
-        wall(a, self);
-        each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst); });
-      }
-      if (zhi) {
-        wall(a, self + step);
-        each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst + step); });
-      }
-      if (zend) {
-        const long back = (b.a2[a] - b.a1[a] + b.ng) * step;
-        wall(a, self - back);
-        each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst - back); });
-      }
+    // wall faces, bit 0 the cell's own, bit 1 its upper one, bit 2 the mirror
+    // image past the low ghosts, and their images along the other axes
+    unsigned walls = b.flag[2 * a] == BNZ_BC_REFLECT && x[a] == b.a1[a] ? 1u : 0u;
+    if (x[a] == b.a2[a]) {
+      if (b.flag[2 * a + 1] == BNZ_BC_REFLECT) walls |= 2u;
+      if (b.end[a] == END_WALL) walls |= 4u;
+    }
+    unsigned o[3] = {m[0], m[1], m[2]};
+    o[a] = 1u;
+    const long step = a == 0 ? 1 : a == 1 ? g.sy : g.sz;
+    const long self = ((long)k * g.nt[1] + j) * g.nt[0] + i;
+#pragma unroll 1
+    for (; walls; walls &= walls - 1) {
+      const int q = __builtin_ctz(walls);
+      const long off = q == 0 ? 0 : q == 1 ? step : -(b.a2[a] - b.a1[a] + b.ng) * step;
+      wall(a, self + off);
+      each_image(b, g, o, i, j, k, [&](long dst, unsigned) { wall(a, dst + off); });
     }
   }
 }
@@ -312,9 +314,7 @@ inline Bnd bnd_of(const bnz_ctx *c) {
   for (int q = 0; q < 6; ++q) b.flag[q] = c->p.bc[q];
   b.ng = c->ng;
   b.dims = c->dims;
-  b.plain = 1;
-  for (int q = 0; q < 2 * c->dims; ++q)
-    if (b.flag[q] == BNZ_BC_REFLECT) b.plain = 0;
+  b.close();
   return b;
 }
 

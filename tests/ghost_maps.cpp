@@ -19,16 +19,13 @@ static void check(const int n[3], int dims, int ng, const int bc[6]) {
   int nt[3];
   b.ng = ng;
   b.dims = dims;
-  b.plain = 1;
   for (int a = 0; a < 3; ++a) {
     nt[a] = g.nt[a] = a < dims ? n[a] + 2 * ng : 1;
     b.a1[a] = a < dims ? ng : 0;
     b.a2[a] = a < dims ? n[a] + ng - 1 : 0;
   }
-  for (int q = 0; q < 6; ++q) {
-    b.flag[q] = bc[q];
-    if (q < 2 * dims && bc[q] == BNZ_BC_REFLECT) b.plain = 0;
-  }
+  for (int q = 0; q < 6; ++q) b.flag[q] = bc[q];
+  b.close();
   g.dims = dims;
   g.sy = nt[0];
   g.sz = nt[0] * nt[1];
