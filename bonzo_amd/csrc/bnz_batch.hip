@@ -485,10 +485,10 @@ void axis_coords(int N, int ind1, int ind2, int nact, double lmin, double lmax, 
 // which tiles waste more than they save.  threads: those of the better tile's
 // stages a cell, the corrector's, which cost twice the predictor's, counted
 // twice.  us per step of 64 boxes of 1e6 cells together, separate / tiles,
-// (threads): 3x1736 209 / 273 (2.4), 4x1562 208 / 251 (2.1), 12x868 206 / 222 (2.0),
-// 5x1420 210 / 233 (1.94), 9x1041 207 / 204 (1.9), 10x976 207 / 187 (1.8), 15x744
-// 204 / 210 (1.7), 1736x3 168 / 177 (1.9), 976x10 167 / 158 (1.6).  FP64 boxes:
-// 3x1736 313 / 331, 12x868 312 / 320, all others faster with tiles.
+// (threads): 3x1736 210 / 257 (2.4), 4x1562 206 / 231 (2.1), 12x868 201 / 205 (2.0),
+// 5x1420 208 / 219 (1.94), 1736x3 166 / 160 (1.9), 9x1041 205 / 194 (1.9), 10x976 205
+// / 180 (1.8), 15x744 200 / 194 (1.7).  FP64 boxes: 3x1736 316 / 332, 12x868 312 /
+// 323, all others faster with tiles.
 constexpr long THIN2_CELLS32 = 1L << 17;
 bool thin_box32(const BoxDev &d) {
   if (d.g.dims != 2) return false;
@@ -496,7 +496,7 @@ bool thin_box32(const BoxDev &d) {
     return tile_threads(d.g.nt, d.L[0], true, e) + 2 * tile_threads(d.g.nt, d.L[1], false, e);
   };
   return std::min(threads(TILE2_SMALL), threads(TILE2_BIG32)) >
-         1.85 * 3. * (double)d.g.nt[0] * d.g.nt[1];
+         1.92 * 3. * (double)d.g.nt[0] * d.g.nt[1];
 }
 
 Box mkbox(int i0, int ni, int j0, int nj, int k0, int nk) {
@@ -921,10 +921,10 @@ int bnz_batch_create(const bnz_params *p, const bnz_box *boxes, int nbox, bnz_ba
   gops.insert(gops.end(), gops2.begin(), gops2.end());
   c->nghost = (long)pairs.size();
   c->ngops = (long)gops.size();
-  // us per step of 64 boxes, small / big tile: FP64 1736x3 263 / 303, 1562x4 250
-  // / 270, 744x15 248 / 260 (the same threads), 1302x6 239 / 242, 36x372 242 / 217
-  // (a sixth more); FP32C 10x976 187 / 245, 30x434 191 / 231, 36x372 170 / 196,
-  // 1562x4 160 / 169 (a sixth more), 60x236 177 / 195 (0.94), 372x36 164 / 147
+  // us per step of 64 boxes, small / big tile: FP64 1736x3 264 / 306, 1562x4 251
+  // / 271, 744x15 248 / 262 (the same threads), 1302x6 240 / 243, 36x372 242 / 218
+  // (a sixth more); FP32C 10x976 180 / 231, 30x434 181 / 212, 36x372 164 / 184,
+  // 1562x4 149 / 156 (a sixth more), 60x236 168 / 180 (0.94), 372x36 159 / 136
   c->tile_small = cells2 <= TILE2_SMALL_CELLS ||
                   (c->f32 ? 10 * small_threads <= 9 * big_threads : small_threads <= big_threads);
   const int *e = c->tile_small ? TILE2_SMALL : big;

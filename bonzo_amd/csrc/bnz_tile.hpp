@@ -400,14 +400,14 @@ constexpr int TILE3[2] = {16, 16};
 // their rounds walk (Tiling3::cost), the separate kernels as long as the grid
 // has cells: columns pay where the cells are at least the given share of the
 // cells that the walked planes have room for.  Thin sides, which leave most of
-// a tile idle, and grids whose last round is nearly empty fall below it.  us per
-// step, separate / columns, over 101 shapes of 3 to 30000 cells a side: no shape
-// is more than 6 % slower than with the better of the two.  share, FP64: 0.40
-// (3x3x30000) 899 / 1464, 0.59 (30x30x1000) 495 / 521, 0.64 (200x16x200) 352 /
-// 360, 0.66 (200x8x300) 321 / 283, 0.87 (128^3) 917 / 731; FMA: 0.53 0.93 times
-// as fast, 0.59 1.02; FP32C: 0.62 (1000x3x1000) 1863 / 2640, 0.64 (5x320x300) 265
-// / 326, 0.71 (96^3) 237 / 261, 0.73 (322x337x33) 1.06 times as fast, 0.74 (112^3)
-// 409 / 410, 0.83 (104^3) 295 / 283.
+// a tile idle, and grids whose last round is nearly empty fall below it.  Over 101
+// shapes of 3 to 30000 cells a side no shape is more than 6 % slower than with the
+// better of the two.  us per step, separate / columns, at that share: FP64 0.40
+// (3x3x30000) 979 / 1454, 0.59 (30x30x1000) 524 / 516, 0.64 (200x16x200) 351 / 359,
+// 0.66 (200x8x300) 326 / 283, 0.84 (128^3) 943 / 732; FMA 0.53 0.93 times as fast,
+// 0.59 1.02; FP32C 0.62 (1000x3x1000) 1984 / 2612, 0.64 (5x320x300) 277 / 324, 0.71
+// (96^3) 244 / 256, 0.73 (322x337x33) 1039 / 965, 0.74 (112^3) 406 / 408, 0.83
+// (104^3) 320 / 277.
 inline bool columns_pay(const bnz_ctx *c) {
   if (c->ncell > STAGE3_MAX_CELLS ||
       c->ncell < (c->f32 ? STAGE3_MIN_CELLS32 : STAGE3_MIN_CELLS64))
@@ -422,9 +422,9 @@ inline bool columns_pay(const bnz_ctx *c) {
 
 // Whether a 2D grid is too thin for tiles: long grids some ten cells across
 // with their ghosts, where a tile's row or column is mostly idle.  us per step,
-// separate / tiles: FP64 200000x3 516 / 536, 3x200000 593 / 560, 4x150000 472 /
-// 424 (FMA 200000x3 503 / 500); FP32C 3x22222 62 / 68, 4x20000 60 / 63, 5x18181
-// 61 / 58, 22222x3 57 / 38 (its tile is wider than high).  Short grids are bound
+// separate / tiles: FP64 200000x3 514 / 542, 3x200000 601 / 561, 4x150000 472 /
+// 424 (FMA 200000x3 504 / 517); FP32C 3x22222 61 / 66, 4x20000 58 / 60, 5x18181
+// 59 / 58, 22222x3 55 / 37 (its tile is wider than high).  Short grids are bound
 // by their launches, of which tiles have fewer (FP32C 3x2000 27 / 22).
 inline bool thin2(const bnz_ctx *c) {
   if (c->f32) return c->nt[0] <= 10 && c->ncell > 1L << 17;
@@ -462,10 +462,9 @@ inline long tile_threads(const int *nt, const Lims &L, bool pred, const int *e) 
 // or neither tile's do and the grid is below TILE2_SMALL_CELLS or covered with
 // four fifths of the threads (a thin grid of 12 rows: 18 with ghosts are 3
 // rows of small tiles, 2 of big).  us per step, FP64, small / big tile (256
-// CUs): 128^2 (230 / 100 workgroups) 19.1 / 20.6, 160^2 (336 / 144) 25.7 / 20.8,
-// 200^2 (525 / 225) 26.8 / 22.0, 300x190 (726 / 308) 28.4 / 29.4, 250^2 (836 /
-// 361) 29.6 / 29.2, 11111x12 62.8 / 77.3, 83333x12 343 / 501 (separate kernels
-// 458).
+// CUs): 128^2 (230 / 100 workgroups) 18.5 / 20.3, 160^2 (336 / 144) 25.1 / 20.5,
+// 200^2 (525 / 225) 25.7 / 21.1, 300x190 (726 / 308) 26.9 / 28.1, 250^2 (836 /
+// 361) 28.0 / 28.0, 11111x12 63 / 77, 83333x12 345 / 495 (separate kernels 449).
 inline bool tile_small64(const bnz_ctx *c, const Lims &L, bool pred) {
   const auto fits = [&](const int *e) {
     return tiling2(c->nt, L, pred, e[0] - 2, e[1] - 2).blocks() <= c->ncu;
@@ -477,10 +476,10 @@ inline bool tile_small64(const bnz_ctx *c, const Lims &L, bool pred) {
              4 * tile_threads(c->nt, L, pred, TILE2_BIG64);
 }
 
-// Whether an FP32C one does, which holds more waves a CU: by cells (200^2 21.6 /
-// 23.9, 250^2 23.4 / 23.3), or where it takes nine tenths of the threads, as on
-// grids that use little of the big tile's rows of 32 (8x14285 45 / 57, 8x107142
-// 216 / 357, separate 305; 10x93750 231 / 305, 12x83333 294 / 292).
+// Whether an FP32C one does, which holds more waves a CU: by cells (200^2 20.9 /
+// 23.4, 250^2 22.5 / 22.6), or where it takes nine tenths of the threads, as on
+// grids that use little of the big tile's rows of 32 (8x14285 45 / 56, 8x107142
+// 202 / 343, separate 305; 10x93750 223 / 295, 12x83333 278 / 283).
 inline bool tile_small32(const bnz_ctx *c, const Lims &L, bool pred) {
   return c->ncell <= TILE2_SMALL_CELLS ||
          10 * tile_threads(c->nt, L, pred, TILE2_SMALL) <=
