@@ -111,7 +111,7 @@ __global__ __launch_bounds__(BLK) void kb_update(const BoxDev *__restrict__ boxe
 // which the caller makes current.  As in the single grid's 2D stages (k_stage2)
 // no flux goes through HBM, and a step is three launches instead of seven: 24
 // FP32C blasts of side 64 .. 320 to t = 0.1 took 93 ms with separate launches
-// and take 76, the copies to and from the host included.
+// and take 71, the copies to and from the host included.
 template <bool PRED, int ORDER, int RS, int TX, int TY>
 __global__ __launch_bounds__(TX *TY, 2) void kb_stage2(
     const BoxDev *__restrict__ boxes, WList wl, BoxState st, Pools p, int fms_ref) {

@@ -448,7 +448,7 @@ void stage32(bnz_ctx *c, int order, const Lims &L) {
   }
 }
 
-// A 2D FP32C step as two launches (as the FP64 stage2_launch): w32, b -> ws32,
+// A 2D FP32C step's stages, a launch each (as the FP64 stage2_launch): w32, b -> ws32,
 // bs32 -> uh, ul, w32 in place and the faces to bs.
 template <bool PRED, int ORDER, int RS, int TX, int TY>
 void stage2_launch32(bnz_ctx *c, const Lims &L) {
@@ -510,7 +510,7 @@ void stage_fused32(bnz_ctx *c, const Lims &L) {
 }
 
 void f32_step_body(bnz_ctx *c) {
-  if (fused_stages(c)) {  // 2D: ghosts and time included
+  if (fused_stages(c)) {  // in 2D the corrector fills the ghosts and advances the time
     if (c->pdt_pending && c->pdt.npart > DT_PARTS_IN_STAGE) flush_dt(c);
     stage_fused32<true, 0>(c, integr_lims(c, 0));
     if (c->order) stage_fused32<false, 1>(c, integr_lims(c, 1));

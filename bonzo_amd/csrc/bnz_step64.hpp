@@ -215,7 +215,7 @@ __global__ __launch_bounds__(BLK) void k_update(Geo g, const double *w0, const d
 // One stage of a 2D grid, a tile per workgroup (stage2_tile).  The predictor
 // finds the step's dt (step_dt); the corrector leaves the CFL partial of its
 // tile, writes the ghosts and advances the time, so that a step is two
-// launches.
+// launches (a third for the dt beyond DT_PARTS_IN_STAGE tiles).
 template <bool PRED, int ORDER, int RS, int TX, int TY>
 __global__ __launch_bounds__(TX *TY, 2) void k_stage2(Geo g, const double *__restrict__ wf,
                                                    const double *__restrict__ bf,
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(NT) void k_tube(Geo g, Bnd bnd, double *w, double *
 // Launches
 // ==========================================================================
 
-// A 2D step as two launches: w, b -> ws, bs -> w, ee (the face buffer the
+// A 2D step's stages, a launch each: w, b -> ws, bs -> w, ee (the face buffer the
 // caller swaps with b; no EMF array is needed here).
 template <bool PRED, int ORDER, int RS, int TX, int TY>
 void stage2_launch(bnz_ctx *c, const Lims &L) {
@@ -443,8 +443,7 @@ void launch_emf(bnz_ctx *c, const double *w, const Lims &L, const char *name) {
 #undef EMF_ARGS
 }
 
-// One VL step after the dt kernels (vanleer.pyx:100-163).
-// we: with emf_fly, the prim the stage's EMFs come from
+// A stage's update of every cell; we: with emf_fly, the prim its EMFs come from.
 void launch_update(bnz_ctx *c, bool pred, const Lims &L, const double *we = nullptr) {
   double *w1 = pred ? c->ws : c->w;
   Box grid;
@@ -575,7 +574,6 @@ void launch_rk3_body(bnz_ctx *c) {
   launch_ghost_step64(c);  // and the time advance
 }
 
-// One VL step after the dt kernels (vanleer.pyx:100-163).
 template <int ORDER, int RS>
 void tube_launch(bnz_ctx *c, int nsteps) {
   const DtFold dtf = take_dt(c);
@@ -609,6 +607,7 @@ void launch_tube(bnz_ctx *c, int nsteps) {
 #undef TUBE
 }
 
+// One VL step after the dt kernels (vanleer.pyx:100-163), or RK3 step.
 void launch_step_body(bnz_ctx *c) {
   if (c->p.tintegr) {
     launch_rk3_body(c);
@@ -616,7 +615,7 @@ void launch_step_body(bnz_ctx *c) {
   }
   Lims L0 = integr_lims(c, 0);
   Lims L1 = integr_lims(c, c->order);
-  if (fused_stages(c)) {  // 2D: ghosts and time included
+  if (fused_stages(c)) {  // in 2D the corrector fills the ghosts and advances the time
     if (c->pdt_pending && c->pdt.npart > DT_PARTS_IN_STAGE) flush_dt(c);
     stage_fused<true, 0>(c, L0);
     if (c->order) stage_fused<false, 1>(c, L1);

@@ -501,9 +501,11 @@ inline long tile_parts(const bnz_ctx *c) {
   return n;
 }
 
-// A pending dt over more partials than this is reduced by a launch of its
-// own (the first step after an upload of a large grid: k_dt_partial leaves
-// one per 256 cells), not by every workgroup of the stage.
+// A pending dt over more partials than this is reduced by a launch of its own,
+// not by every workgroup of the stage: on the first step after an upload of a
+// large grid (k_dt_partial leaves one per 256 cells), and on every step of a 2D
+// grid of more tiles than that (FP64 from about 900^2 on: 1024^2 leaves 5476),
+// which then is three launches (k_dt_final takes 5 us there).
 constexpr int DT_PARTS_IN_STAGE = 4096;
 
 }  // namespace bnz

@@ -247,11 +247,13 @@ enum {
 // those of stage2_tile, except that no ghosts are written; every thread must
 // call it.
 //   Bound by FP64 VALU issue: the separate kernels move about 35 GB per 256^3
-// step (24 flux words a cell and stage), this moves 16 and leaves the solves,
-// 1.46 times those of the grid (rims, and the two planes more of each run).
-// The SIMDs issue VALU work 0.61 (predictor) and 0.68 (corrector) of the
-// time, the rest being load and barrier waits of two waves per SIMD.
-// Measured at 256^3 (FMA; us per launch, predictor / corrector): separate
+// step (24 flux words a cell and stage), this 16.4 (7.4 + 9.0, reads that the
+// MALL serves included) and leaves the solves, 1.46 times those of the grid (rims,
+// and the two planes more of each run).  The SIMDs issue VALU work 0.64 (predictor)
+// and 0.73 (corrector) of the time, the rest being load and barrier waits of two
+// waves per SIMD, at 1917 and 2360 us a launch (FMA, 256^3; IEEE 0.72 and 0.79 at
+// 2141 and 2742).
+// How it got there (FMA, one after another on one card; us per launch): separate
 // kernels 3330 / 3760; one 32 x 16 workgroup a CU with every face's stencil
 // loaded 2560 / 3740, two of 16 x 16 2410 / 3000 (a workgroup's barrier waits
 // then overlap the other's solves), plane above loaded ahead and half slopes
