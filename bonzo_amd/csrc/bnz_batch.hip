@@ -560,12 +560,12 @@ void b_update(bnz_batch *c) {
   if (wl.hi != wl.lo)
     hipLaunchKernelGGL((kb_update<PRED>), dim3(grid_for(wl.hi - wl.lo, c->cap[TU])), dim3(BLK), 0,
                        c->stream, c->boxes, wl, c->S, c->P, c->p.dt_fms_ref);
-  const int order = PRED ? 0 : c->order, rs = c->p.rsolver;
-  if (order == 0) {
+  const int rs = c->p.rsolver;
+  if (PRED || c->order == 0) {
     if (rs == BNZ_RS_HLLD) b_stages<PRED, 0, BNZ_RS_HLLD>(c);
     else if (rs == BNZ_RS_HLLT) b_stages<PRED, 0, BNZ_RS_HLLT>(c);
     else b_stages<PRED, 0, BNZ_RS_HLL>(c);
-  } else {
+  } else if constexpr (!PRED) {
     if (rs == BNZ_RS_HLLD) b_stages<PRED, 1, BNZ_RS_HLLD>(c);
     else if (rs == BNZ_RS_HLLT) b_stages<PRED, 1, BNZ_RS_HLLT>(c);
     else b_stages<PRED, 1, BNZ_RS_HLL>(c);

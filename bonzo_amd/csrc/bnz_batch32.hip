@@ -425,7 +425,7 @@ void updates(bnz_batch *c) {
   if (PRED || c->order == 0) {
     if (hlld) stages<PRED, 0, BNZ_RS_HLLD>(c);
     else stages<PRED, 0, BNZ_RS_HLL>(c);
-  } else {
+  } else if constexpr (!PRED) {
     if (hlld) stages<PRED, 1, BNZ_RS_HLLD>(c);
     else stages<PRED, 1, BNZ_RS_HLL>(c);
   }
