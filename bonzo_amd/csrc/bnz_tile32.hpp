@@ -88,11 +88,11 @@ constexpr int tile2_lds32() {
 }
 
 // One FP32C stage over one 2D tile (stage2_tile).  The fluxes come from the
-// stage's FP32 prim wf and faces bf; ap / ac as in the separate updates.  As
-// there the corrector updates the active cells only and writes their ghosts:
-// it reads the words of its own active cells, which no other tile writes, and
-// wf, bf and ac.b, which no corrector writes.  ng counts the guarded faces of
-// the cells the tile owns.
+// stage's FP32 prim wf and faces bf; ap / ac as in the separate updates.  Like
+// the FP64 tile's, the corrector updates the active cells only and writes their
+// ghosts: it reads the words of its own active cells, which no other tile
+// writes, and wf, bf and ac.b, which no corrector writes.  ng counts the guarded
+// faces of the cells the tile owns.
 template <bool PRED, int ORDER, int RS, int TX, int TY, typename BF, class DT>
 __device__ __forceinline__ double stage2_tile32(const Geo &g, const float *__restrict__ wf,
                                                 const BF *__restrict__ bf, const Pred32 &ap,
